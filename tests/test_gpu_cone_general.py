@@ -182,3 +182,50 @@ def test_volume_of_more_than_2pow29_voxels(oracle):
     e32 = rel_l2(oracle.siddon_cone_bp(g, y, *hg, prec='f'), ref)
     _say('bp rel-L2 %.2e (the reference arithmetic in FP32: %.2e)' % (e, e32))
     assert e < 1e-3 and e < 0.1 * e32
+
+
+@pytest.mark.parametrize('case', ['ragged', 'flipped_rows', 'fine_rows', 'more_rows', 'fine_columns', 'axis_parallel', 'truncated',
+                                  'batch'])
+def test_bp_plane_form(oracle, tuning, case):
+    """The plane form of the backprojector (one crossing ray per voxel plane and
+    detector column) against the oracle, and against the candidate windows
+    (cone_bp_planes 2): grids that end inside a block, det_v pointing down,
+    several rows and several columns per voxel, rays along the axes (no jitter,
+    odd panel, source on a voxel plane), planes outside the panel, and volumes
+    sharing the geometry.  'fine_rows' has more rows per voxel than the plane
+    form takes and keeps the windows.  The rays of 'axis_parallel' run within
+    voxel faces, where the voxel they count for is a tie that both forms decide
+    alike and the oracle otherwise: compared with the windows only."""
+    from ctprojector_amd.phantom import circular_cone_geometry
+    from ctprojector_amd.projector.numpy import cone
+    from ctprojector_amd.projector.numpy.ct_projector import ct_projector
+    kw = dict(nx=23, ny=19, nz=37, dx=1.0, dy=1.0, dz=1.0, cx=0.4, cy=-0.3, cz=0.7, nu=44, nv=45, du=1.7, dv=1.7,
+              off_u=0.2, off_v=-0.4, dsd=300.0, dso=180.0)
+    jitter, B = 1.0, 1
+    if case == 'fine_rows':
+        kw.update(dz=1.5, nz=21, dv=0.8, nv=90)
+    if case == 'more_rows':
+        kw.update(dz=1.5, nz=21, dv=1.1, nv=70)
+    if case == 'fine_columns':
+        kw.update(du=0.6, nu=120)
+    if case == 'axis_parallel':
+        kw.update(nx=24, ny=24, nz=24, cx=0.0, cy=0.0, cz=0.0, nu=45, off_u=0.0, off_v=0.0)
+        jitter = 0.0
+    if case == 'truncated':
+        kw.update(nv=7, nu=15, off_v=3.0)
+    if case == 'batch':
+        B = 3
+    g = Geo(**kw)
+    z = 0.0 if case == 'axis_parallel' else 6.0
+    geo = circular_cone_geometry(12, 180.0, 300.0, -z, z, jitter=jitter, seed=5)
+    if case == 'flipped_rows':
+        geo.det_v = -geo.det_v
+    args = (geo.det_center, geo.det_u, geo.det_v, geo.src)
+    y = np.random.default_rng(8).uniform(size=[B, 12, g.nv, g.nu]).astype(np.float32)
+    p = g.to(ct_projector())
+    a = cone.siddon_bp_arbitrary(p, y, *args)
+    tuning('cone_bp_planes', 2)
+    b = cone.siddon_bp_arbitrary(p, y, *args)
+    e, d = rel_l2(a, oracle.siddon_cone_bp(g, y, *args)), rel_l2(a, b)
+    _say(case, 'plane form against the oracle %.2e, against the windows %.2e' % (e, d))
+    assert d < TOL and (e < TOL or case == 'axis_parallel')
