@@ -64,6 +64,33 @@ __device__ inline float med_clamp(float x, float s, float e) { return med3_f(x, 
 __device__ inline float min_f(float a, float b) { return med3_f(a, b, -3.0e38f); }
 __device__ inline float max_f(float a, float b) { return med3_f(a, b, 3.0e38f); }
 
+#ifdef __HIPCC__
+// atan(t) for |t| <= 0.7 ('narrow', uniform across the wavefront), else through
+// the library: t + t z P(z), z = t^2, with P the degree-6 Chebyshev
+// interpolant of (atan(t)/t - 1)/z on [0, 0.5] (within 1 ulp; 9 instructions
+// where the general function reduces its argument with a division).
+__device__ inline float fan_atan(float t, bool narrow) {
+    if (!narrow) return atanf(t);
+    const float z = t * t;
+    float p = -0.0178704802f;
+    p = fmaf(p, z, 0.0521920919f);
+    p = fmaf(p, z, -0.083692804f);
+    p = fmaf(p, z, 0.109958887f);
+    p = fmaf(p, z, -0.142766684f);
+    p = fmaf(p, z, 0.199997291f);
+    p = fmaf(p, z, -0.333333313f);
+    return fmaf(t, p * z, t);
+}
+
+// Whether every pixel of the grid is seen from the source (dso from the
+// rotation centre) within atan 0.7 of the central ray: a point at distance r
+// from the centre is at most asin(r / dso) off it.
+__device__ inline bool fan_narrow(const Grid& g, float dso) {
+    const float x = fabsf(g.cx) + 0.5f * (float)g.nx * g.dx, y = fabsf(g.cy) + 0.5f * (float)g.ny * g.dy;
+    return __builtin_amdgcn_readfirstlane(x * x + y * y < 0.32f * dso * dso ? 1 : 0) != 0;
+}
+#endif
+
 inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 
 // Read-only data loaded through the constant address space: wave-uniform

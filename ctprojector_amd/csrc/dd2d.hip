@@ -33,6 +33,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace ctp {
@@ -85,32 +86,46 @@ static void hard_switch(std::vector<DDView>& v) {
 // ---------------------------------------------------------------------------
 // layout transforms
 // ---------------------------------------------------------------------------
-// planes P[c][y][x] (c < C)  ->  O[major * rs + minor * cs + c] with (major,
-// minor) = (y, x) (xmajor=false) or (x, y) (xmajor=true); rs >= minor extent *
-// cs is the row stride; channels >= C are written as zero.
-// Block (bx, by, bz) = (32 pixels of a row, 32 channels, row y) of the copy.
+// planes P[c][y][x] (c < C)  ->  O[major * rs + (pad + minor) * cs + c] with
+// (major, minor) = (y, x) (xmajor=false) or (x, y) (xmajor=true); rs >=
+// (minor extent + 2 pad) * cs is the row stride; channels >= C and the pad
+// pixels at both ends of a row are written as zero.
+// Block (bx, by, bz) = (32 pixels of a row, 32 channels, row y) of the copy,
+// counted from the pads (pad_blocks_x / _y of them).
 __device__ inline void to_channel_last_block(float* __restrict__ out, const float* __restrict__ in, int C, int cs,
-                                             int nx, int ny, bool xmajor, size_t rs, int bx, int by, int bz) {
+                                             int nx, int ny, bool xmajor, size_t rs, int pad, int bx, int by, int bz) {
     __shared__ float tile[32][33];
-    const int x0 = bx * 32, c0 = by * 32, y = bz;
+    const int px = xmajor ? 0 : pad, py = xmajor ? pad : 0;
+    const int x0 = bx * 32 - px, c0 = by * 32, y = bz - py;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8
     for (int k = ty; k < 32; k += 8) {
         const int c = c0 + k, x = x0 + tx;
-        tile[k][tx] = (c < C && x < nx) ? in[((size_t)c * ny + y) * nx + x] : 0.f;
+        tile[k][tx] = (c < C && x >= 0 && x < nx && y >= 0 && y < ny) ? in[((size_t)c * ny + y) * nx + x] : 0.f;
     }
     __syncthreads();
+    if (cs < 32) {
+        // few channels: consecutive lanes write consecutive floats
+        for (int i = threadIdx.x; i < 32 * cs; i += 256) {
+            const int k = i / cs, c = i - k * cs, x = x0 + k;
+            if (x < nx + px) {
+                const size_t at = xmajor ? (size_t)x * rs + (size_t)bz * cs : (size_t)y * rs + (size_t)(x + px) * cs;
+                out[at + c] = tile[c][k];
+            }
+        }
+        return;
+    }
     for (int k = ty; k < 32; k += 8) {
         const int x = x0 + k, c = c0 + tx;
-        if (x < nx && c < cs) {
-            const size_t at = xmajor ? (size_t)x * rs + (size_t)y * cs : (size_t)y * rs + (size_t)x * cs;
+        if (x < nx + px && c < cs) {
+            const size_t at = xmajor ? (size_t)x * rs + (size_t)bz * cs : (size_t)y * rs + (size_t)(x + px) * cs;
             out[at + c] = tile[tx][k];
         }
     }
 }
 
 __global__ __launch_bounds__(256) void to_channel_last(float* __restrict__ out, const float* __restrict__ in, int C,
-                                                       int cs, int nx, int ny, bool xmajor, size_t rs) {
-    to_channel_last_block(out, in, C, cs, nx, ny, xmajor, rs, blockIdx.x, blockIdx.y, blockIdx.z);
+                                                       int cs, int nx, int ny, bool xmajor, size_t rs, int pad) {
+    to_channel_last_block(out, in, C, cs, nx, ny, xmajor, rs, pad, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // ---------------------------------------------------------------------------
@@ -125,34 +140,245 @@ struct FPRow {        // one output row (b, iv) of a channel chunk
 
 // Footprint of one line [x1, x2] (index units, unclamped) on a pixel row of
 // length n: the reference's IntegralBoxX (cuda/cudaMath.cu:533-565) divided by
-// (x2 - x1), applied to a channel vector at 'row' (stride cs between pixels).
-// XC: the channel after the chunk (the next chunk's first slice, for the z
-// interpolation across chunks) is accumulated too.
-template <int CH, bool XC>
-__device__ inline void dd_line(float* acc, const float* __restrict__ row, int cs, float x1, float x2, int n, float scale) {
+// (x2 - x1): pixels i1 .. i2 (none if i1 > i2) weighted by their overlap with
+// [a, b] times inv.
+struct Footprint {
+    float a, b, inv;
+    int i1, i2;
+    __device__ inline float weight(int i) const { return (fminf(b, (float)(i + 1)) - fmaxf(a, (float)i)) * inv; }
+};
+
+__device__ inline Footprint footprint(float x1, float x2, int n, float scale) {
     const float lo = min_f(x1, x2), hi = max_f(x1, x2);
-    const float a = med_clamp(lo, 0.f, (float)n), b = med_clamp(hi, 0.f, (float)n);
-    if (!(b > a)) return;
-    const float inv = fast_div(scale, hi - lo);
-    const int i1 = min((int)a, n - 1), i2 = min((int)b, n - 1);
-    for (int i = i1; i <= i2; i++) {
-        const float w = (fminf(b, (float)(i + 1)) - fmaxf(a, (float)i)) * inv;
-        const float* p = row + (size_t)i * cs;
-        if constexpr (CH % 4 == 0) {
+    Footprint f;
+    f.a = med_clamp(lo, 0.f, (float)n);
+    f.b = med_clamp(hi, 0.f, (float)n);
+    f.inv = fast_div(scale, hi - lo);
+    f.i1 = min((int)f.a, n - 1);
+    f.i2 = f.b > f.a ? min((int)f.b, n - 1) : -1;
+    return f;
+}
+
+// a pixel's channel vector (CH channels; XC: and the one after)
+template <int CH, bool XC>
+__device__ inline void load_pixel(float* q, const float* __restrict__ p) {
+    if constexpr (CH % 4 == 0) {
 #pragma unroll
-            for (int j = 0; j < CH; j += 4) {
-                const float4 q = *reinterpret_cast<const float4*>(p + j);
-                acc[j] = fmaf(w, q.x, acc[j]);
-                acc[j + 1] = fmaf(w, q.y, acc[j + 1]);
-                acc[j + 2] = fmaf(w, q.z, acc[j + 2]);
-                acc[j + 3] = fmaf(w, q.w, acc[j + 3]);
+        for (int j = 0; j < CH; j += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(p + j);
+            q[j] = v.x; q[j + 1] = v.y; q[j + 2] = v.z; q[j + 3] = v.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < CH; j++) q[j] = p[j];
+    }
+    if constexpr (XC) q[CH] = p[CH];
+}
+
+// The footprints f[0 .. U-1] of U rows (or views), each on its own row of
+// pixels (stride cs), applied in order to the channel accumulators.  A
+// footprint is mostly one or two pixels: the first two of all U rows are
+// loaded before any is used, so that U rows' memory latencies overlap (a lane
+// that takes its rows one by one waits for memory at each).  Lanes load and
+// add only the pixels their footprint touches.
+template <int CH, bool XC, int U>
+__device__ inline void apply_footprints(float* acc, const Footprint* f, const float* const* row, int cs) {
+    constexpr int N = CH + (XC ? 1 : 0);
+    float q0[U][N], q1[U][N];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const float* __restrict__ p = row[u] + (size_t)f[u].i1 * cs;
+        if (f[u].i2 >= f[u].i1) load_pixel<CH, XC>(q0[u], p);
+        if (f[u].i2 > f[u].i1) load_pixel<CH, XC>(q1[u], p + cs);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        if (f[u].i2 >= f[u].i1) {
+            const float w = f[u].weight(f[u].i1);
+#pragma unroll
+            for (int j = 0; j < N; j++) acc[j] = fmaf(w, q0[u][j], acc[j]);
+        }
+        if (f[u].i2 > f[u].i1) {
+            const float w = f[u].weight(f[u].i1 + 1);
+#pragma unroll
+            for (int j = 0; j < N; j++) acc[j] = fmaf(w, q1[u][j], acc[j]);
+        }
+        for (int i = f[u].i1 + 2; i <= f[u].i2; i++) {
+            const float w = f[u].weight(i);
+            float q[N];
+            load_pixel<CH, XC>(q, row[u] + (size_t)i * cs);
+#pragma unroll
+            for (int j = 0; j < N; j++) acc[j] = fmaf(w, q[j], acc[j]);
+        }
+    }
+}
+
+// Rows (or views) a lane takes together: as many as keep the loaded channels
+// within 32 registers.
+template <int CH>
+constexpr int footprint_batch() { return CH >= 16 ? 1 : CH == 8 ? 2 : 4; }
+
+// Whether a column passes an image of n pixels a row on one side through all
+// rows t0 .. t1 - 1 (its ends are linear in the row; 0.01 pixel for rounding),
+// and its largest width there.
+__device__ inline bool fp_passes(int t0, int t1, int n, float r1, float o1, float q1, float r2, float o2, float q2,
+                                 float& wide) {
+    const float ta = (float)t0 + 0.5f, tb = (float)t1 - 0.5f;
+    const float a1 = fmaf(r1, ta - o1, q1), a2 = fmaf(r2, ta - o2, q2);
+    const float b1 = fmaf(r1, tb - o1, q1), b2 = fmaf(r2, tb - o2, q2);
+    wide = fmaxf(fabsf(a1 - a2), fabsf(b1 - b2));
+    return fmaxf(fmaxf(a1, a2), fmaxf(b1, b2)) <= -0.01f || fminf(fminf(a1, a2), fminf(b1, b2)) >= (float)n + 0.01f;
+}
+
+// Rows t0 .. t1 - 1 of one trace of a column: the column's lines at row
+// coordinate t + 0.5 are fmaf(r1, t + 0.5 - o1, q1) and fmaf(r2, t + 0.5 - o2, q2)
+// on rows of n pixels (row stride rs floats).
+template <int CH, bool XC>
+__device__ inline void fp_trace_rows(float* acc, const float* __restrict__ img, size_t rs, int cs, int t0, int t1,
+                                     int n, float r1, float o1, float q1, float r2, float o2, float q2, float norm) {
+    constexpr int U = footprint_batch<CH>();
+    for (int t = t0; t < t1; t += U) {
+        Footprint f[U];
+        const float* row[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const float tt = (float)(t + u) + 0.5f;
+            f[u] = footprint(fmaf(r1, tt - o1, q1), fmaf(r2, tt - o2, q2), n, norm);
+            if (t + u >= t1) f[u].i2 = -1;
+            row[u] = img + (size_t)(t + u < t1 ? t + u : t) * rs;
+        }
+        apply_footprints<CH, XC, U>(acc, f, row, cs);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Window form of the one-lane kernels (up to 4 channels)
+// ---------------------------------------------------------------------------
+// With few channels the footprint arithmetic outweighs the channels' multiply-
+// adds, and the walk above issues about 55 (FP) and 106 (fan BP) VALU
+// instructions per footprint at one channel, which is what bounds it.  Where
+// no footprint of the wavefront is wider than K - 1 pixels it meets at most K
+// pixels, from floor(lo) on: rows carry kPad zero pixels at both ends, so a
+// footprint needs no clamping to the row, no loop and no masks, and its K
+// weights are differences of consecutive pixel edges limited to hi.  Pixels a
+// footprint does not meet must not count even where they are not finite: up
+// to 2 channels their weight 0 is multiplied by the legacy product (0 * x = 0
+// for every x); at 4 they are read from a pad.  Both leave the sums as the
+// walk's, up to rounding.  Measured at 512^2 / 984 views / 888 columns, 1 and
+// 4 slices: fan FP 748 -> 306 and 914 -> 540 us, fan BP 804 -> 438 and 849 ->
+// 565, parallel FP 727 -> 249 and 875 -> 500, parallel BP 622 -> 333 and 747
+// -> 494.
+constexpr int kPad = 4;
+
+// 0 * x = 0 for every x
+__device__ inline float mul_legacy(float a, float b) {
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// K pixels of one row (or of one view's detector row), rows[0] the first pad
+// pixel: weights w[K] (w[0] first) of the footprint between lo and hi, and the
+// channel vectors.
+template <int CH, int K>
+struct Window {
+    float w[K], q[K][CH], scale;
+    __device__ inline void load(const float* __restrict__ row, float lo, float hi, float nf) {
+        scale = __builtin_amdgcn_rcpf(max_f(hi - lo, 1e-30f));
+        const float fl = floorf(lo);
+        float edge = lo;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const float next = k + 1 < K ? min_f(hi, fl + (float)(k + 1)) : hi;
+            w[k] = next - edge;
+            edge = next;
+        }
+        // byte offset from the row's first pad; footprints beyond the row read pads
+        const unsigned off = (unsigned)__mul24((int)med_clamp(fl, -(float)kPad, nf), 4 * CH) + 4u * kPad * CH;
+        const char* __restrict__ rb = reinterpret_cast<const char*>(row);
+        if constexpr (CH <= 2) {
+            typedef float vec __attribute__((ext_vector_type(K * CH), aligned(4 * CH)));
+            const vec v = *reinterpret_cast<const vec*>(rb + off);
+#pragma unroll
+            for (int i = 0; i < K * CH; i++) q[i / CH][i % CH] = v[i];
+        } else {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const unsigned o = k == 0 || w[k] > 0.f ? off + 4u * CH * k : 0u;
+                load_pixel<CH, false>(q[k], reinterpret_cast<const float*>(rb + o));
+            }
+        }
+    }
+    // acc += s times the footprint's integral over its width
+    __device__ inline void add(float* acc, float s) const {
+        const float ws = scale * s;
+        if constexpr (CH <= 2) {
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                float t = mul_legacy(w[K - 1], q[K - 1][j]);
+#pragma unroll
+                for (int k = K - 2; k > 0; k--) t += mul_legacy(w[k], q[k][j]);
+                acc[j] = fmaf(ws, fmaf(w[0], q[0][j], t), acc[j]);
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < CH; j++) acc[j] = fmaf(w, p[j], acc[j]);
+            for (int k = 0; k < K; k++)
+#pragma unroll
+                for (int j = 0; j < CH; j++) acc[j] = fmaf(w[k] * ws, q[k][j], acc[j]);
         }
-        if constexpr (XC) acc[CH] = fmaf(w, p[CH], acc[CH]);
     }
+};
+
+constexpr int kWindowBatch = 4;   // rows (views) a lane takes together
+
+// Rows t0 .. t1 - 1 of one trace of a column (fp_trace_rows) on padded rows:
+// img the first row's first pad, rs floats per row.
+template <int CH, int K>
+__device__ inline void fp_trace_window(float* acc, const float* __restrict__ img, int rs, int t0, int t1, int n,
+                                       float r1, float o1, float q1, float r2, float o2, float q2) {
+    constexpr int U = kWindowBatch;
+    const float nf = (float)n;
+    auto rows = [&](int t, auto count) {
+        constexpr int N = decltype(count)::value;
+        Window<CH, K> W[N];
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const float tt = (float)(t + u) + 0.5f;
+            const float e1 = fmaf(r1, tt - o1, q1), e2 = fmaf(r2, tt - o2, q2);
+            W[u].load(img + (size_t)(t + u) * rs, min_f(e1, e2), max_f(e1, e2), nf);
+        }
+#pragma unroll
+        for (int u = 0; u < N; u++) W[u].add(acc, 1.f);
+    };
+    int t = t0;
+    for (; t + U <= t1; t += U) rows(t, std::integral_constant<int, U>{});
+    for (; t < t1; t++) rows(t, std::integral_constant<int, 1>{});
+}
+
+// One trace of a column for up to 4 channels, 32 rows at a time: the window
+// form where the footprints allow it, else the walk.  A footprint's ends are
+// linear in the row, so those of the chunk's end rows bound them; columns that
+// pass the image on one side through the whole chunk read pads only, and a
+// chunk that all of them pass is left out.  (In the fan beam the outer columns
+// of oblique views are several pixels wide, most of them beside the image.)
+template <int CH>
+__device__ inline void fp_trace_small(float* acc, const float* __restrict__ img, int rs, int tbeg, int tend, int n,
+                                      float r1, float o1, float q1, float r2, float o2, float q2, float norm) {
+    float part[CH];
+#pragma unroll
+    for (int j = 0; j < CH; j++) part[j] = 0.f;
+    for (int t0 = tbeg; t0 < tend; t0 += 32) {
+        const int t1 = min(t0 + 32, tend);
+        float wide;
+        const bool past = fp_passes(t0, t1, n, r1, o1, q1, r2, o2, q2, wide);
+        if (!__any(!past)) continue;   // uniform, as the choices below
+        if (past) wide = 0.f;
+        if (!__any(!(wide < 0.999f))) fp_trace_window<CH, 2>(part, img, rs, t0, t1, n, r1, o1, q1, r2, o2, q2);
+        else if (!__any(!(wide < 1.999f))) fp_trace_window<CH, 3>(part, img, rs, t0, t1, n, r1, o1, q1, r2, o2, q2);
+        else fp_trace_rows<CH, false>(part, img + kPad * CH, (size_t)rs, CH, t0, t1, n, r1, o1, q1, r2, o2, q2, 1.f);
+    }
+#pragma unroll
+    for (int j = 0; j < CH; j++) acc[j] = fmaf(norm, part[j], acc[j]);
 }
 
 // The two edge rays of detector column iu in image index coordinates: from
@@ -191,13 +417,14 @@ __device__ inline float fp_cell_edges(int iu, const DDView& V, const Grid& g, co
     return a;
 }
 
-// A block is 128 lanes: 128 >> lseg detector columns times 2^lseg segments of
-// the image rows (lseg 0 or 1: one segment per wavefront, so the row loop
-// stays scalar).  Each lane integrates its column's footprint over its
+// VPB 1: a block is 128 lanes, 128 >> lseg detector columns times 2^lseg
+// segments of the image rows (lseg 0 or 1); VPB -4 and -8: 64 columns times 4
+// or 8 segments (lseg 2 or 3).  A segment is a wavefront's, so the row loop
+// stays scalar.  Each lane integrates its column's footprint over its
 // segment; the segments' accumulators are summed in LDS in a fixed order.
-// Splitting the rows doubles the waves of launches with few columns, views
+// Splitting the rows multiplies the waves of launches with few columns, views
 // and channel chunks (2D slices) so that they can hide the row gathers'
-// latency.
+// latency, and shortens each lane's chain of rows.
 // VPB > 1: a block is VPB wavefronts of VPB consecutive views over the same
 // 64 columns (one segment): the views' footprints on a row nearly coincide, so
 // the wavefronts of a block read the same image lines at about the same time
@@ -208,9 +435,10 @@ template <int CH, bool FAN, bool XC, int VPB>
 __device__ inline void dd_fp_block(
         float* __restrict__ prj, const float* __restrict__ imgY, const float* __restrict__ imgX,
         const DDView* __restrict__ views, const FPRow* __restrict__ rows, const int* __restrict__ row_start, int cs,
-        const Grid& g, const Det& d, int nview, float dsd, float dso, bool force, int lseg, int bx, int by, int bz) {
-    __shared__ float lds[VPB > 1 ? 64 * VPB : 128][CH + 2];
-    const int lcol = VPB > 1 ? 6 : 7 - lseg;
+        const Grid& g, const Det& d, int nview, float dsd, float dso, bool force, int lseg, int pad, int bx, int by,
+        int bz) {
+    __shared__ float lds[VPB == 1 ? 128 : 64 * (VPB < 0 ? -VPB : VPB)][CH + 2];
+    const int lcol = VPB != 1 ? 6 : 7 - lseg;
     const int col = threadIdx.x & ((1 << lcol) - 1);
     const int seg = VPB > 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> lcol);   // uniform per wavefront
     const int nseg = VPB > 1 ? 1 : 1 << lseg;
@@ -234,28 +462,28 @@ __device__ inline void dd_fp_block(
             const float r1 = (d1.x - s1.x) / (d1.y - s1.y);
             const float r2 = (d2.x - s2.x) / (d2.y - s2.y);
             const float norm = V.wx * g.dy / fabsf(cosf(V.deg - a));
-            // rows addressed from the int extents (a 64-bit row-stride argument
-            // instead measured 8% slower at 512x512x32)
-            const int ye = (int)(((long)g.ny * (seg + 1)) >> lseg);
-            for (int iy = (int)(((long)g.ny * seg) >> lseg); iy < ye; iy++) {
-                const float yy = (float)iy + 0.5f;
-                const float x1 = fmaf(r1, yy - s1.y, s1.x);
-                const float x2 = fmaf(r2, yy - s2.y, s2.x);
-                dd_line<CH, XC>(acc, bY + (size_t)iy * g.nx * cs, cs, x1, x2, g.nx, norm);
-            }
+            const int t0 = (int)(((long)g.ny * seg) >> lseg), t1 = (int)(((long)g.ny * (seg + 1)) >> lseg);
+            bool done = false;
+            if constexpr (CH <= 4 && !XC)
+                if (pad > 0) {
+                    fp_trace_small<CH>(acc, bY, (g.nx + 2 * kPad) * CH, t0, t1, g.nx, r1, s1.y, s1.x, r2, s2.y, s2.x, norm);
+                    done = true;
+                }
+            if (!done) fp_trace_rows<CH, XC>(acc, bY, (size_t)g.nx * cs, cs, t0, t1, g.nx, r1, s1.y, s1.x, r2, s2.y, s2.x, norm);
         }
         if (V.flags & 2) {
             // trace along x, cuda/distanceDriven2DBoxInt.cu:74-98
             const float r1 = (d1.y - s1.y) / (d1.x - s1.x);
             const float r2 = (d2.y - s2.y) / (d2.x - s2.x);
             const float norm = (1.f - V.wx) * g.dx / fabsf(sinf(V.deg - a));
-            const int xe = (int)(((long)g.nx * (seg + 1)) >> lseg);
-            for (int ix = (int)(((long)g.nx * seg) >> lseg); ix < xe; ix++) {
-                const float xx = (float)ix + 0.5f;
-                const float y1 = fmaf(r1, xx - s1.x, s1.y);
-                const float y2 = fmaf(r2, xx - s2.x, s2.y);
-                dd_line<CH, XC>(acc, bX + (size_t)ix * g.ny * cs, cs, y1, y2, g.ny, norm);
-            }
+            const int t0 = (int)(((long)g.nx * seg) >> lseg), t1 = (int)(((long)g.nx * (seg + 1)) >> lseg);
+            bool done = false;
+            if constexpr (CH <= 4 && !XC)
+                if (pad > 0) {
+                    fp_trace_small<CH>(acc, bX, (g.ny + 2 * kPad) * CH, t0, t1, g.ny, r1, s1.x, s1.y, r2, s2.x, s2.y, norm);
+                    done = true;
+                }
+            if (!done) fp_trace_rows<CH, XC>(acc, bX, (size_t)g.ny * cs, cs, t0, t1, g.ny, r1, s1.x, s1.y, r2, s2.x, s2.y, norm);
         }
     }
 #pragma unroll
@@ -284,11 +512,11 @@ __device__ inline void dd_fp_block(
 }
 
 template <int CH, bool FAN, bool XC, int VPB>
-__global__ __launch_bounds__(VPB > 1 ? 64 * VPB : 128) void dd_fp_kernel(
+__global__ __launch_bounds__(VPB == 1 ? 128 : 64 * (VPB < 0 ? -VPB : VPB)) void dd_fp_kernel(
         float* __restrict__ prj, const float* __restrict__ imgY, const float* __restrict__ imgX,
         const DDView* __restrict__ views, const FPRow* __restrict__ rows, const int* __restrict__ row_start, int cs,
-        Grid g, Det d, int nview, float dsd, float dso, bool force, int lseg) {
-    dd_fp_block<CH, FAN, XC, VPB>(prj, imgY, imgX, views, rows, row_start, cs, g, d, nview, dsd, dso, force, lseg,
+        Grid g, Det d, int nview, float dsd, float dso, bool force, int lseg, int pad) {
+    dd_fp_block<CH, FAN, XC, VPB>(prj, imgY, imgX, views, rows, row_start, cs, g, d, nview, dsd, dso, force, lseg, pad,
                                   blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
@@ -726,6 +954,7 @@ struct DDFPSetup {
     int lseg = 0;   // direct kernel: 2^lseg row segments per column
     int lpc = 1;    // lanes per detector column (> 1: dd_fp_split_kernel)
     bool xc = true; // pixels carry the channel after the chunk
+    int pad = 0;    // zero pixels at both ends of the copies' rows (window form)
     long rsY = 0, rsX = 0;   // row strides (floats) of the y-major and x-major copies (n * cs)
 };
 
@@ -781,7 +1010,7 @@ static DDFPSetup dd_fp_setup(const std::vector<DDView>& views, int B, const Grid
     const int wcap = 65536 / (2 * CHP * 4);   // two row buffers in 64 KiB of LDS
     // the direct kernel is the default (measured faster at 512x512x32: the
     // staged kernel's prefetch registers spill)
-    const bool want_lds = allow_lds && tuning_get("dd_fp_mode", 1) == 2 && s.groups.size() <= 65535;
+    const bool want_lds = allow_lds && tuning_get("dd_fp_mode", 0) == 2 && s.groups.size() <= 65535;
     const double wneed = want_lds ? fp_stage_width(views, s.groups, g, d, dsd, dso, fan) + 6.0 : 1e300;
     s.use_lds = want_lds && wneed <= (double)wcap;
     s.wmax = s.use_lds ? (int)std::ceil(wneed) : 0;
@@ -815,21 +1044,41 @@ static DDFPSetup dd_fp_setup(const std::vector<DDView>& views, int B, const Grid
     // where split lanes are asked for (2 lanes 0.27 ms there)
     const int forced = tuning_get("dd_fp_segments", 0);
     const int rows_min = std::min(g.nx, g.ny);
-    const int seg_rule = (rows_min / 2 >= 32 && 2L * ceil_div(d.nu, 128) * nview * nchunk < 4096) ? 1 : 0;
+    int seg_rule = (rows_min / 2 >= 32 && 2L * ceil_div(d.nu, 128) * nview * nchunk < 4096) ? 1 : 0;
+    // more segments while the launch stays under 2048 waves (2 per SIMD) and
+    // a segment keeps at least 12 rows
+    if (seg_rule == 1 && CH <= 8)
+        while (seg_rule < 3 && ((long)ceil_div(d.nu, 64) * nview * nchunk << seg_rule) < 2048 &&
+               rows_min >> (seg_rule + 1) >= 12)
+            seg_rule++;
     const int lpc = lpc_req > 0 ? std::min(lpc_req, std::max(CH / 4, 1))
                                 : tuning_get("dd_fp_lanes_per_column", CH >= 16 ? CH / 8 : 1);
     const bool split = !s.xc && forced != 2 && (CH >= 16 || seg_rule == 0) && (CH == 8 || CH == 16 || CH == 32) &&
                        (lpc == 2 || lpc == 4 || lpc == 8) && CH % (4 * lpc) == 0;
     int lseg = split ? 0 : seg_rule;
-    if (forced == 1 || forced == 2) lseg = forced - 1;
+    if (forced == 1 || forced == 2) lseg = forced - 1;   // (3 and 4: 4 and 8 segments, up to 8 channels)
+    if ((forced == 3 || forced == 4) && CH <= 8 && !split) lseg = forced - 1;
     s.lseg = lseg;
     if (split) {
         s.lpc = lpc;
         s.cs = CH;
     }
-    s.rsY = (long)g.nx * s.cs;
-    s.rsX = (long)g.ny * s.cs;
+    // up to 4 channels the one-lane kernel runs the window form (dd_fp_mode 1
+    // keeps the pixel-by-pixel walk); at 8 the third pixel's 32 bytes cost more
+    // than the arithmetic saves (512^2 / 984 views, fan: walk 1.28 ms, window 1.64)
+    if (!split && !s.xc && !s.use_lds && CH <= 4 && s.cs == CH && tuning_get("dd_fp_mode", 0) == 0 &&
+        (long)(std::max(g.nx, g.ny) + 2 * kPad) * CH < (1 << 21))
+        s.pad = kPad;
+    s.rsY = (long)(g.nx + 2 * s.pad) * s.cs;
+    s.rsX = (long)(g.ny + 2 * s.pad) * s.cs;
     return s;
+}
+
+// Block form of the one-lane kernel (its VPB): 4 or 8 row segments, else views
+// per block (tv, one segment) or 1.
+static int fp_block_form(int lseg, int tv) {
+    if (lseg >= 2) return -(1 << lseg);
+    return lseg == 0 && (tv == 2 || tv == 4) ? tv : 1;
 }
 
 struct DDFPDev {
@@ -852,12 +1101,14 @@ static void dd_fp_run(const DDFPSetup& s, const DDFPDev& t, float* prj, const fl
     dim3 tb(256);
     if (s.needY) {
         TimedLaunch tt("dd_transpose", stream);
-        to_channel_last<<<dim3(ceil_div(g.nx, 32), ceil_div(cs, 32), g.ny), tb, 0, stream>>>(imgY, img, C, cs, g.nx, g.ny, false, (size_t)s.rsY);
+        to_channel_last<<<dim3(ceil_div(g.nx + 2 * s.pad, 32), ceil_div(cs, 32), g.ny), tb, 0, stream>>>(
+            imgY, img, C, cs, g.nx, g.ny, false, (size_t)s.rsY, s.pad);
         CTP_LAUNCH_CHECK();
     }
     if (s.needX) {
         TimedLaunch tt("dd_transpose", stream);
-        to_channel_last<<<dim3(ceil_div(g.nx, 32), ceil_div(cs, 32), g.ny), tb, 0, stream>>>(imgX, img, C, cs, g.nx, g.ny, true, (size_t)s.rsX);
+        to_channel_last<<<dim3(ceil_div(g.nx, 32), ceil_div(cs, 32), g.ny + 2 * s.pad), tb, 0, stream>>>(
+            imgX, img, C, cs, g.nx, g.ny, true, (size_t)s.rsX, s.pad);
         CTP_LAUNCH_CHECK();
     }
     if (s.use_lds) {
@@ -900,17 +1151,19 @@ static void dd_fp_run(const DDFPSetup& s, const DDFPDev& t, float* prj, const fl
     }
     const int lseg = s.lseg;
     const int tv = tuning_get("dd_fp_views_per_block", 4);
-    const int vpb = (lseg == 0 && (tv == 2 || tv == 4)) ? tv : 1;
-    dim3 grid(ceil_div(d.nu, 128 >> lseg), nview, nchunk), block(128);
+    const int vpb = fp_block_form(lseg, tv);
+    dim3 grid(ceil_div(d.nu, lseg > 0 ? 64 : 128), nview, nchunk), block(vpb < 0 ? -64 * vpb : 128);
     if (vpb > 1) {
         grid = dim3(ceil_div(d.nu, 64), ceil_div(nview, vpb), nchunk);
         block = dim3(64 * vpb);
     }
     TimedLaunch tt(fan ? "dd_fan_fp" : "dd_par_fp", stream);
 #define CTP_FP_LAUNCH(N, F, X) \
-    if (vpb == 4) dd_fp_kernel<N, F, X, 4><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg); \
-    else if (vpb == 2) dd_fp_kernel<N, F, X, 2><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg); \
-    else dd_fp_kernel<N, F, X, 1><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg)
+    if (vpb == -4) { if constexpr (N <= 8) dd_fp_kernel<N, F, X, -4><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg, s.pad); } \
+    else if (vpb == -8) { if constexpr (N <= 8) dd_fp_kernel<N, F, X, -8><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg, s.pad); } \
+    else if (vpb == 4) dd_fp_kernel<N, F, X, 4><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg, s.pad); \
+    else if (vpb == 2) dd_fp_kernel<N, F, X, 2><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg, s.pad); \
+    else dd_fp_kernel<N, F, X, 1><<<grid, block, 0, stream>>>(prj, imgY, imgX, dviews, drows, dstart, cs, g, d, nview, dsd, dso, force, lseg, s.pad)
 #define CTP_FP_CASE(N)                                                                                          \
     case N:                                                                                                     \
         if (fan) { if (s.xc) CTP_FP_LAUNCH(N, true, true); else CTP_FP_LAUNCH(N, true, false); }               \
@@ -1027,19 +1280,20 @@ void dd2d_fp_noalloc(float* prj, const float* img, const float* deg_host, int B,
 // clamped linear interpolation between rows of InterpolateXY
 // (cuda/distanceDriven2DBranchless.cu:444-447, cuda/cudaMath.cu:227-260); the
 // u-interpolation of the prefix sums there is the exact box integral used below.
-// Block (bx, by, bz) = (32 columns, 32 channels, view).
+// Rows of pad zero cells, the detector's, pad zero cells.
+// Block (bx, by, bz) = (32 columns from the first pad on, 32 channels, view).
 __device__ inline void dd_bp_prep_block(float* __restrict__ sino, const float* __restrict__ prj,
                                         const DDView* __restrict__ views, const SliceRow* __restrict__ slice_row, int C,
                                         int cs, int nz, const Det& d, int nview, float dx, float dy, bool fan,
-                                        bool preweight, int bx, int by, int bz) {
+                                        bool preweight, int pad, int bx, int by, int bz) {
     __shared__ float tile[32][33];
-    const int u0 = bx * 32, c0 = by * 32, view = bz;
+    const int u0 = bx * 32 - pad, c0 = by * 32, view = bz;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     const DDView V = preweight ? views[view] : DDView{};
     for (int k = ty; k < 32; k += 8) {
         const int c = c0 + k, u = u0 + tx;
         float val = 0.f;
-        if (c < C && u < d.nu) {
+        if (c < C && u >= 0 && u < d.nu) {
             const int b = c / nz, z = c - b * nz;
             const SliceRow R = slice_row[z];
             if (R.r0 >= 0) {
@@ -1057,15 +1311,15 @@ __device__ inline void dd_bp_prep_block(float* __restrict__ sino, const float* _
     __syncthreads();
     for (int k = ty; k < 32; k += 8) {
         const int u = u0 + k, c = c0 + tx;
-        if (u < d.nu && c < cs) sino[((size_t)view * d.nu + u) * cs + c] = tile[tx][k];
+        if (u < d.nu + pad && c < cs) sino[((size_t)view * (d.nu + 2 * pad) + u + pad) * cs + c] = tile[tx][k];
     }
 }
 
 __global__ __launch_bounds__(256) void dd_bp_prep_kernel(float* __restrict__ sino, const float* __restrict__ prj,
                                                          const DDView* __restrict__ views, const SliceRow* __restrict__ slice_row,
                                                          int C, int cs, int nz, Det d, int nview, float dx, float dy,
-                                                         bool fan, bool preweight) {
-    dd_bp_prep_block(sino, prj, views, slice_row, C, cs, nz, d, nview, dx, dy, fan, preweight, blockIdx.x, blockIdx.y,
+                                                         bool fan, bool preweight, int pad) {
+    dd_bp_prep_block(sino, prj, views, slice_row, C, cs, nz, d, nview, dx, dy, fan, preweight, pad, blockIdx.x, blockIdx.y,
                      blockIdx.z);
 }
 
@@ -1073,36 +1327,76 @@ void slices_to_channel_last(float* sino, const float* prj, const SliceRow* rows_
                             const Det& d, int nview, hipStream_t stream) {
     TimedLaunch t("fbp_bp_prep", stream);
     dd_bp_prep_kernel<<<dim3(ceil_div(d.nu, 32), ceil_div(cs, 32), nview), 256, 0, stream>>>(
-        sino, prj, nullptr, rows_dev, C, cs, nz, d, nview, 1.f, 1.f, false, false);
+        sino, prj, nullptr, rows_dev, C, cs, nz, d, nview, 1.f, 1.f, false, false, 0);
     CTP_LAUNCH_CHECK();
 }
 
-// Detector footprint [a1, a2] (cell units, unclamped) of a pixel applied to the
-// channel vectors of one view: IntegralBoxX over a detector row divided by
-// (a2 - a1), cuda/distanceDriven2DBoxInt.cu:375-383.
-template <int CH>
-__device__ inline void dd_cells(float* acc, const float* __restrict__ base, int cs, float a1, float a2, int n, float scale) {
-    const float lo = min_f(a1, a2), hi = max_f(a1, a2);
-    const float a = med_clamp(lo, 0.f, (float)n), b = med_clamp(hi, 0.f, (float)n);
-    if (!(b > a)) return;
-    const float inv = fast_div(scale, hi - lo);
-    const int i1 = min((int)a, n - 1), i2 = min((int)b, n - 1);
-    for (int i = i1; i <= i2; i++) {
-        const float w = (fminf(b, (float)(i + 1)) - fmaxf(a, (float)i)) * inv;
-        const float* p = base + (size_t)i * cs;
-        if constexpr (CH % 4 == 0) {
+// Views vbeg .. vend - 1 of the backprojection of pixel centre (xc, yc) in the
+// window form (up to 4 channels; sino rows padded by kPad cells): the pixel's
+// detector footprints, mostly 0.7 to 1.4 cells wide, meet at most 3 cells.
+// Views of wider footprints are walked cell by cell.
+template <int CH, bool FAN>
+__device__ inline void bp_views_window(float* acc, const float* __restrict__ sino, const DDView* __restrict__ views,
+                                       int vbeg, int vend, float xc, float yc, const Grid& g, const Det& d, float rdu,
+                                       float dso, bool fbp, bool narrow) {
+    constexpr int U = kWindowBatch;
+    const float half = (float)d.nu / 2.0f, nf = (float)d.nu, mid = half - d.off_u;
+    const size_t vstride = (size_t)(d.nu + 2 * kPad) * CH;
+    const float hx = g.dx / 2.0f, hy = g.dy / 2.0f;
+    // (main axis tr: the footprint is the projection of the pixel's extent along x (0) or y (1))
+    auto batch = [&](int v0, auto count, int tr) {
+        constexpr int N = decltype(count)::value;
+        float lo[N], hi[N], scale[N];
+        bool on[N], wide = false, some = false;
 #pragma unroll
-            for (int j = 0; j < CH; j += 4) {
-                const float4 q = *reinterpret_cast<const float4*>(p + j);
-                acc[j] = fmaf(w, q.x, acc[j]);
-                acc[j + 1] = fmaf(w, q.y, acc[j + 1]);
-                acc[j + 2] = fmaf(w, q.z, acc[j + 2]);
-                acc[j + 3] = fmaf(w, q.w, acc[j + 3]);
+        for (int u = 0; u < N; u++) {
+            const DDView V = const_load(views, v0 + u);
+            const float c = V.c, s = V.s;
+            float u1, u2;
+            on[u] = FAN || (V.flags & (1 << tr)) != 0;   // uniform
+            some = some || on[u];
+            if (FAN) {
+                // cuda/distanceDriven2DBoxInt.cu:362-391 and GetProjectionOnDetector (Utils.cu:96-102)
+                const bool ym = (V.flags & 4) != 0;
+                const float num = fmaf(xc, c, yc * s), den = fmaf(yc, c, -(xc * s)) + dso;
+                const float hn = ym ? hx * c : hy * s, hd = ym ? -hx * s : hy * c;
+                u1 = fmaf(-fan_atan(fast_div(num - hn, den - hd), narrow), rdu, mid);
+                u2 = fmaf(-fan_atan(fast_div(num + hn, den + hd), narrow), rdu, mid);
+                scale[u] = fbp ? fast_div(dso * dso, fmaf(num, num, den * den)) : 1.f;
+            } else {
+                // cuda/distanceDriven2DBoxInt.cu:439-493 (blended main axes)
+                const float num = fmaf(xc, c, yc * s), hn = tr == 0 ? hx * c : hy * s;
+                u1 = fmaf(hn - num, rdu, mid);
+                u2 = fmaf(-hn - num, rdu, mid);
+                scale[u] = tr == 0 ? V.wx : 1.f - V.wx;
             }
-        } else {
-#pragma unroll
-            for (int j = 0; j < CH; j++) acc[j] = fmaf(w, p[j], acc[j]);
+            lo[u] = min_f(u1, u2);
+            hi[u] = max_f(u1, u2);
+            wide = wide || (on[u] && !(hi[u] - lo[u] < 1.999f));
         }
+        if (!some) return;
+        if (__any(wide)) {
+#pragma unroll
+            for (int u = 0; u < N; u++) {
+                if (!on[u]) continue;
+                const Footprint f = footprint(lo[u], hi[u], d.nu, scale[u]);
+                const float* row = sino + (size_t)(v0 + u) * vstride + kPad * CH;
+                apply_footprints<CH, false, 1>(acc, &f, &row, CH);
+            }
+            return;
+        }
+        Window<CH, 3> W[N];
+#pragma unroll
+        for (int u = 0; u < N; u++) W[u].load(sino + (size_t)(v0 + u) * vstride, lo[u], hi[u], nf);
+#pragma unroll
+        for (int u = 0; u < N; u++)
+            if (on[u]) W[u].add(acc, scale[u]);
+    };
+#pragma unroll
+    for (int tr = 0; tr < (FAN ? 1 : 2); tr++) {
+        int v = vbeg;
+        for (; v + U <= vend; v += U) batch(v, std::integral_constant<int, U>{}, tr);
+        for (; v < vend; v++) batch(v, std::integral_constant<int, 1>{}, tr);
     }
 }
 
@@ -1127,36 +1421,65 @@ __device__ inline void dd_bp_block(float* __restrict__ img, float* __restrict__ 
     for (int j = 0; j < CH; j++) acc[j] = 0.f;
     const float half = (float)d.nu / 2.0f;
     const size_t vstride = (size_t)d.nu * cs;
-    for (int view = vbeg; view < vend; view++) {
-        const DDView V = views[view];
-        const float c = V.c, s = V.s;
-        const float* __restrict__ base = sino + view * vstride + c0;
+    const bool narrow = FAN && fan_narrow(g, dso);
+    const float rdu = 1.f / d.du;
+    if constexpr (CH <= 4) {
+        bp_views_window<CH, FAN>(acc, sino, views, vbeg, vend, xc, yc, g, d, rdu, dso, fbp, narrow);
+        store_bp_result<CH>(img, part, acc, grp, c0, C, (size_t)g.nx * g.ny, (size_t)iy * g.nx + ix);
+        return;
+    }
+    // Detector footprints [u1, u2] (cell units, unclamped) of the pixel, applied
+    // to the channel vectors of the views: IntegralBoxX over a detector row
+    // divided by (u2 - u1), cuda/distanceDriven2DBoxInt.cu:375-383
+    constexpr int U = footprint_batch<CH>();
+    for (int v0 = vbeg; v0 < vend; v0 += U) {
         if (FAN) {
-            // cuda/distanceDriven2DBoxInt.cu:362-391 and GetProjectionOnDetector (Utils.cu:96-102)
-            float p1x, p1y, p2x, p2y;
-            if (V.flags & 4) { p1x = x1; p1y = yc; p2x = x2; p2y = yc; }
-            else { p1x = xc; p1y = y1; p2x = xc; p2y = y2; }
-            const float a1 = atanf(fast_div(p1x * c + p1y * s, -p1x * s + p1y * c + dso));
-            const float a2 = atanf(fast_div(p2x * c + p2y * s, -p2x * s + p2y * c + dso));
-            const float u1 = -(fast_div(a1, d.du) + d.off_u) + half;
-            const float u2 = -(fast_div(a2, d.du) + d.off_u) + half;
-            float scale = 1.f;
-            if (fbp) {
-                const float rx = xc * c + yc * s, ry = -xc * s + yc * c;
-                scale = fast_div(dso * dso, rx * rx + (dso + ry) * (dso + ry));
+            Footprint f[U];
+            const float* row[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int view = min(v0 + u, vend - 1);
+                const DDView V = const_load(views, view);
+                const float c = V.c, s = V.s;
+                // cuda/distanceDriven2DBoxInt.cu:362-391 and GetProjectionOnDetector (Utils.cu:96-102)
+                float p1x, p1y, p2x, p2y;
+                if (V.flags & 4) { p1x = x1; p1y = yc; p2x = x2; p2y = yc; }
+                else { p1x = xc; p1y = y1; p2x = xc; p2y = y2; }
+                const float a1 = fan_atan(fast_div(p1x * c + p1y * s, -p1x * s + p1y * c + dso), narrow);
+                const float a2 = fan_atan(fast_div(p2x * c + p2y * s, -p2x * s + p2y * c + dso), narrow);
+                const float u1 = -(a1 * rdu + d.off_u) + half;
+                const float u2 = -(a2 * rdu + d.off_u) + half;
+                float scale = 1.f;
+                if (fbp) {
+                    const float rx = xc * c + yc * s, ry = -xc * s + yc * c;
+                    scale = fast_div(dso * dso, rx * rx + (dso + ry) * (dso + ry));
+                }
+                f[u] = footprint(u1, u2, d.nu, scale);
+                if (v0 + u >= vend) f[u].i2 = -1;
+                row[u] = sino + view * vstride + c0;
             }
-            dd_cells<CH>(acc, base, cs, u1, u2, d.nu, scale);
+            apply_footprints<CH, false, U>(acc, f, row, cs);
         } else {
             // cuda/distanceDriven2DBoxInt.cu:439-493 (blended main axes)
-            if (V.flags & 1) {
-                const float u1 = -(fast_div(x1 * c + yc * s, d.du) + d.off_u) + half;
-                const float u2 = -(fast_div(x2 * c + yc * s, d.du) + d.off_u) + half;
-                dd_cells<CH>(acc, base, cs, u1, u2, d.nu, V.wx);
-            }
-            if (V.flags & 2) {
-                const float u1 = -(fast_div(xc * c + y1 * s, d.du) + d.off_u) + half;
-                const float u2 = -(fast_div(xc * c + y2 * s, d.du) + d.off_u) + half;
-                dd_cells<CH>(acc, base, cs, u1, u2, d.nu, 1.f - V.wx);
+#pragma unroll
+            for (int tr = 0; tr < 2; tr++) {
+                Footprint f[U];
+                const float* row[U];
+                bool any = false;
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int view = min(v0 + u, vend - 1);
+                    const DDView V = const_load(views, view);
+                    const float c = V.c, s = V.s;
+                    const bool on = (V.flags & (1 << tr)) != 0 && v0 + u < vend;
+                    any = any || on;
+                    const float u1 = -((tr == 0 ? x1 * c + yc * s : xc * c + y1 * s) * rdu + d.off_u) + half;
+                    const float u2 = -((tr == 0 ? x2 * c + yc * s : xc * c + y2 * s) * rdu + d.off_u) + half;
+                    f[u] = footprint(u1, u2, d.nu, tr == 0 ? V.wx : 1.f - V.wx);
+                    if (!on) f[u].i2 = -1;
+                    row[u] = sino + view * vstride + c0;
+                }
+                if (any) apply_footprints<CH, false, U>(acc, f, row, cs);   // uniform
             }
         }
     }
@@ -1210,6 +1533,8 @@ __device__ inline void dd_bp_split_block(float* __restrict__ img, float* __restr
         // lane s of a pixel evaluates the footprint of view v0 + s; the pixel's
         // lanes read each view's footprint from it
         const int lead = lane & ~(LPC - 1);
+        const bool narrow = fan_narrow(g, dso);
+        const float rdu = 1.f / d.du;
         for (int v0 = vbeg; v0 < vend; v0 += LPC) {
             float mu1 = 0.f, mu2 = 0.f, msc = 1.f;
             if (v0 + sub < vend) {
@@ -1219,10 +1544,10 @@ __device__ inline void dd_bp_split_block(float* __restrict__ img, float* __restr
                 float p1x, p1y, p2x, p2y;
                 if (V.flags & 4) { p1x = x1; p1y = yc; p2x = x2; p2y = yc; }
                 else { p1x = xc; p1y = y1; p2x = xc; p2y = y2; }
-                const float a1 = atanf(fast_div(p1x * c + p1y * s, -p1x * s + p1y * c + dso));
-                const float a2 = atanf(fast_div(p2x * c + p2y * s, -p2x * s + p2y * c + dso));
-                mu1 = -(fast_div(a1, d.du) + d.off_u) + half;
-                mu2 = -(fast_div(a2, d.du) + d.off_u) + half;
+                const float a1 = fan_atan(fast_div(p1x * c + p1y * s, -p1x * s + p1y * c + dso), narrow);
+                const float a2 = fan_atan(fast_div(p2x * c + p2y * s, -p2x * s + p2y * c + dso), narrow);
+                mu1 = -(a1 * rdu + d.off_u) + half;
+                mu2 = -(a2 * rdu + d.off_u) + half;
                 if (fbp) {
                     const float rx = xc * c + yc * s, ry = -xc * s + yc * c;
                     msc = fast_div(dso * dso, rx * rx + (dso + ry) * (dso + ry));
@@ -1326,8 +1651,10 @@ void reduce_parts(float* img, const float* part, int groups, size_t n, hipStream
 
 struct DDBPSetup {
     int C = 0, CH = 1, nchunk = 1, cs = 0, groups = 1, vpg = 1;
+    int pad = 0;   // zero cells at both ends of the weighted projections' rows (window form)
     bool fbp = false;
     std::vector<SliceRow> srow;
+    size_t sino_floats(const Det& d, int nview) const { return (size_t)nview * (d.nu + 2 * pad) * cs; }
 };
 
 static DDBPSetup dd_bp_setup(int B, const Grid& g, const Det& d, int nview, int type) {
@@ -1339,6 +1666,7 @@ static DDBPSetup dd_bp_setup(int B, const Grid& g, const Det& d, int nview, int 
     s.CH = pick_ch(s.C);
     s.nchunk = ceil_div(s.C, s.CH);
     s.cs = s.nchunk * s.CH;
+    s.pad = s.CH <= 4 ? kPad : 0;   // the kernel's own rule (dd_bp_block)
     // detector rows of each slice, cuda/distanceDriven2DBoxInt.cu:340-350
     s.srow.resize(g.nz);
     for (int z = 0; z < g.nz; z++) {
@@ -1370,8 +1698,8 @@ static void dd_bp_run(const DDBPSetup& s, const DDView* dviews, const SliceRow* 
     const bool fbp = s.fbp;
     {
         TimedLaunch t("dd_bp_prep", stream);
-        dd_bp_prep_kernel<<<dim3(ceil_div(d.nu, 32), ceil_div(cs, 32), nview), 256, 0, stream>>>(
-            sino, prj, dviews, dsrow, C, cs, g.nz, d, nview, g.dx, g.dy, fan, !fbp);
+        dd_bp_prep_kernel<<<dim3(ceil_div(d.nu + 2 * s.pad, 32), ceil_div(cs, 32), nview), 256, 0, stream>>>(
+            sino, prj, dviews, dsrow, C, cs, g.nz, d, nview, g.dx, g.dy, fan, !fbp, s.pad);
         CTP_LAUNCH_CHECK();
     }
     TimedLaunch tb(fan ? "dd_fan_bp" : "dd_par_bp", stream);
@@ -1567,10 +1895,10 @@ void dd2d_bp(float* img, const float* prj, const float* deg_host, int B, const G
     const size_t npix = (size_t)g.nx * g.ny;
     Workspace& ws = workspace_for(stream);
     Plan pl;
-    pl.add<float>((size_t)nview * d.nu * s.cs);
+    pl.add<float>(s.sino_floats(d, nview));
     if (s.groups > 1) pl.add<float>((size_t)s.groups * s.C * npix);
     ws.reserve(pl.bytes);
-    float* sino = ws.take_n<float>((size_t)nview * d.nu * s.cs);
+    float* sino = ws.take_n<float>(s.sino_floats(d, nview));
     float* part = s.groups > 1 ? ws.take_n<float>((size_t)s.groups * s.C * npix) : nullptr;
     dd_bp_run(s, pin.t->views, pin.t->srow, sino, part, img, prj, g, d, nview, dso, fan, stream);
     CTP_CHECK(hipStreamSynchronize(stream));   // the tables stay pinned until the work is done
@@ -1646,10 +1974,11 @@ void rows_to_channel_last(float* q, const float* prj, const int* cstart, const C
 
 // detector column coordinate (column iu spans [iu, iu + 1]) of a physical point
 template <bool FAN>
-__device__ inline float adj_ucoord(float px, float py, float c, float s, const Det& d, float dso) {
+__device__ inline float adj_ucoord(float px, float py, float c, float s, const Det& d, float rdu, float dso,
+                                   bool narrow) {
     const float half = (float)d.nu / 2.0f;
-    if (FAN) return -(atanf((px * c + py * s) / (-px * s + py * c + dso)) / d.du + d.off_u) + half;
-    return -((px * c + py * s) / d.du + d.off_u) + half;
+    if (FAN) return -(fan_atan(fast_div(px * c + py * s, -px * s + py * c + dso), narrow) * rdu + d.off_u) + half;
+    return -((px * c + py * s) * rdu + d.off_u) + half;
 }
 
 template <int CH, bool FAN>
@@ -1667,6 +1996,8 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
     const float xa = ((float)ix - g.nx / 2.f) * g.dx + g.cx, xb = xa + g.dx;
     const float ya = ((float)iy - g.ny / 2.f) * g.dy + g.cy, yb = ya + g.dy;
     const float xc = xa + g.dx / 2, yc = ya + g.dy / 2;
+    const float rdu = 1.f / d.du;
+    const bool narrow = FAN && fan_narrow(g, dso);
     float acc[CH];
 #pragma unroll
     for (int j = 0; j < CH; j++) acc[j] = 0.f;
@@ -1679,8 +2010,8 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
             if (!(V.flags & (1 << tr))) continue;
             // the pixel's interval on its traced row: [ix, ix+1] at y = iy + 0.5 (tr 0)
             // or [iy, iy+1] at x = ix + 0.5 (tr 1), in index units
-            const float ua = tr == 0 ? adj_ucoord<FAN>(xa, yc, V.c, V.s, d, dso) : adj_ucoord<FAN>(xc, ya, V.c, V.s, d, dso);
-            const float ub = tr == 0 ? adj_ucoord<FAN>(xb, yc, V.c, V.s, d, dso) : adj_ucoord<FAN>(xc, yb, V.c, V.s, d, dso);
+            const float ua = tr == 0 ? adj_ucoord<FAN>(xa, yc, V.c, V.s, d, rdu, dso, narrow) : adj_ucoord<FAN>(xc, ya, V.c, V.s, d, rdu, dso, narrow);
+            const float ub = tr == 0 ? adj_ucoord<FAN>(xb, yc, V.c, V.s, d, rdu, dso, narrow) : adj_ucoord<FAN>(xc, yb, V.c, V.s, d, rdu, dso, narrow);
             // candidate columns: those whose span [k, k+1] meets [ua, ub],
             // widened by 1e-3 column for the difference between this FP32
             // projection and the forward projector's FP32 edge lines (about
@@ -1915,7 +2246,7 @@ DDPlan* dd_plan_create(const float* deg_host, int B, const Grid& g, const Det& d
     Plan ps;
     ps.add<float>((size_t)g.ny * p->fp.rsY);
     ps.add<float>((size_t)g.nx * p->fp.rsX);
-    ps.add<float>((size_t)nview * d.nu * p->bp.cs);
+    ps.add<float>(p->bp.sino_floats(d, nview));
     ps.add<float>(p->bp.groups > 1 ? (size_t)p->bp.groups * p->bp.C * npix : 0);
     ps.add<float>((size_t)nview * d.nu * p->adj.cs);
     ps.add<float>(p->adj.groups > 1 ? (size_t)p->adj.groups * p->adj.C * npix : 0);
@@ -1924,7 +2255,7 @@ DDPlan* dd_plan_create(const float* deg_host, int B, const Grid& g, const Det& d
     auto carve_f = [&q](size_t n) { float* r = reinterpret_cast<float*>(q); q += (n * sizeof(float) + 255) / 256 * 256; return r; };
     p->imgY = carve_f((size_t)g.ny * p->fp.rsY);
     p->imgX = carve_f((size_t)g.nx * p->fp.rsX);
-    p->bp_sino = carve_f((size_t)nview * d.nu * p->bp.cs);
+    p->bp_sino = carve_f(p->bp.sino_floats(d, nview));
     p->bp_part = p->bp.groups > 1 ? carve_f((size_t)p->bp.groups * p->bp.C * npix) : nullptr;
     p->adj_G = carve_f((size_t)nview * d.nu * p->adj.cs);
     p->adj_part = p->adj.groups > 1 ? carve_f((size_t)p->adj.groups * p->adj.C * npix) : nullptr;
@@ -2002,9 +2333,9 @@ struct DDJobDev {
     Det d;
     int nview, fan;
     float dsd, dso;
-    int fC, fcs, nrow, lseg, force, needY, needX;   // forward
-    int bC, bcs, nchunk, groups, vpg, fbp;          // backprojection
-    int tr_gx, tr_gy;      // channel-last copies: tr_gx x tr_gy x ny blocks per copy
+    int fC, fcs, nrow, lseg, fpad, force, needY, needX;   // forward
+    int bC, bcs, bpad, nchunk, groups, vpg, fbp;    // backprojection
+    int tr_gx, tr_xx, tr_gy;   // channel-last copies: tr_gx x tr_gy x ny blocks (y-major), tr_xx x tr_gy x (ny + 2 fpad)
     int fp_gx, fp_gy;      // forward projection (third grid dimension: channel chunks)
     int pr_gx, pr_gy;      // weighted projections (third: views)
     int bp_gx, bp_gy;      // backprojection (third: chunks x view groups)
@@ -2040,9 +2371,10 @@ __global__ __launch_bounds__(256) void dd_batch_copy_kernel(DD_BATCH_ARGS) {
         const int per = J.tr_gx * J.tr_gy * J.g.ny;
         const bool xmajor = !J.needY || l >= per;
         const int m = (J.needY && xmajor) ? l - per : l;
-        const int bx = m % J.tr_gx, t = m / J.tr_gx;
+        const int gx = xmajor ? J.tr_xx : J.tr_gx;
+        const int bx = m % gx, t = m / gx;
         to_channel_last_block(xmajor ? J.imgX : J.imgY, J.img, J.fC, J.fcs, J.g.nx, J.g.ny, xmajor,
-                              (size_t)(xmajor ? J.rsX : J.rsY), bx, t % J.tr_gy, t / J.tr_gy);
+                              (size_t)(xmajor ? J.rsX : J.rsY), J.fpad, bx, t % J.tr_gy, t / J.tr_gy);
     }
 }
 
@@ -2056,12 +2388,12 @@ __global__ __launch_bounds__(256) void dd_batch_fp_split_kernel(DD_BATCH_ARGS) {
 }
 
 template <int CH, bool FAN, bool XC, int VPB>
-__global__ __launch_bounds__(VPB > 1 ? 64 * VPB : 128) void dd_batch_fp_kernel(DD_BATCH_ARGS) {
+__global__ __launch_bounds__(VPB == 1 ? 128 : 64 * (VPB < 0 ? -VPB : VPB)) void dd_batch_fp_kernel(DD_BATCH_ARGS) {
     DD_BATCH_LOOP {
         DD_BATCH_JOB;
         const int t = l / J.fp_gx;
         dd_fp_block<CH, FAN, XC, VPB>(J.prj, J.imgY, J.imgX, J.views, J.rows, J.start, J.fcs, J.g, J.d, J.nview,
-                                      J.dsd, J.dso, J.force != 0, J.lseg, l % J.fp_gx, t % J.fp_gy, t / J.fp_gy);
+                                      J.dsd, J.dso, J.force != 0, J.lseg, J.fpad, l % J.fp_gx, t % J.fp_gy, t / J.fp_gy);
     }
 }
 
@@ -2082,7 +2414,7 @@ __global__ __launch_bounds__(256) void dd_batch_prep_kernel(DD_BATCH_ARGS) {
         DD_BATCH_JOB;
         const int t = l / J.pr_gx;
         dd_bp_prep_block(J.sino, J.prj, J.views, J.srow, J.bC, J.bcs, J.g.nz, J.d, J.nview, J.g.dx, J.g.dy,
-                         J.fan != 0, J.fbp == 0, l % J.pr_gx, t % J.pr_gy, t / J.pr_gy);
+                         J.fan != 0, J.fbp == 0, J.bpad, l % J.pr_gx, t % J.pr_gy, t / J.pr_gy);
     }
 }
 
@@ -2217,7 +2549,7 @@ void DDBatchPlan::Impl::setup_jobs() {
         const long rs_max = std::max(widest.rsY, fs.rsY), rx_max = std::max(widest.rsX, fs.rsX);
         J.imgY = fs.needY ? alloc<float>(mem, ny * rs_max) : nullptr;
         J.imgX = fs.needX ? alloc<float>(mem, nx * rx_max) : nullptr;
-        J.sino = alloc<float>(mem, (size_t)S.nview * S.d.nu * bs.cs);
+        J.sino = alloc<float>(mem, bs.sino_floats(S.d, S.nview));
         J.part = bs.groups > 1 ? alloc<float>(mem, (size_t)bs.groups * bs.C * npix) : nullptr;
         DDView* dv = alloc<DDView>(mem, S.nview);
         FPRow* dr = alloc<FPRow>(mem, fs.rows.size());
@@ -2253,6 +2585,16 @@ static const void* dd_launch_kernel(const DDLaunch& L) {
     case DDL_FP:
 #define CTP_K(N)                                                                                               \
     if (L.ch == N) {                                                                                           \
+        if constexpr (N <= 8) {                                                                                \
+            if (L.vpb == -4) return L.fan ? (L.xc ? reinterpret_cast<const void*>(dd_batch_fp_kernel<N, true, true, -4>) \
+                                                  : reinterpret_cast<const void*>(dd_batch_fp_kernel<N, true, false, -4>)) \
+                                          : (L.xc ? reinterpret_cast<const void*>(dd_batch_fp_kernel<N, false, true, -4>) \
+                                                  : reinterpret_cast<const void*>(dd_batch_fp_kernel<N, false, false, -4>)); \
+            if (L.vpb == -8) return L.fan ? (L.xc ? reinterpret_cast<const void*>(dd_batch_fp_kernel<N, true, true, -8>) \
+                                                  : reinterpret_cast<const void*>(dd_batch_fp_kernel<N, true, false, -8>)) \
+                                          : (L.xc ? reinterpret_cast<const void*>(dd_batch_fp_kernel<N, false, true, -8>) \
+                                                  : reinterpret_cast<const void*>(dd_batch_fp_kernel<N, false, false, -8>)); \
+        }                                                                                                      \
         if (L.vpb == 4) return L.fan ? (L.xc ? reinterpret_cast<const void*>(dd_batch_fp_kernel<N, true, true, 4>) \
                                              : reinterpret_cast<const void*>(dd_batch_fp_kernel<N, true, false, 4>)) \
                                      : (L.xc ? reinterpret_cast<const void*>(dd_batch_fp_kernel<N, false, true, 4>) \
@@ -2320,17 +2662,19 @@ void DDBatchPlan::Impl::layout() {
         const DDFPSetup fs = dd_fp_setup(views[j], S.B, S.g, S.d, S.nview, S.dsd, S.dso, S.type, S.fan, false, fp_lpc);
         fps.push_back(fs);
         const DDBPSetup& bs = bps[j];
-        J.fC = fs.C; J.fcs = fs.cs; J.nrow = (int)fs.rows.size(); J.lseg = fs.lseg; J.force = fs.force ? 1 : 0;
+        J.fC = fs.C; J.fcs = fs.cs; J.nrow = (int)fs.rows.size(); J.lseg = fs.lseg; J.fpad = fs.pad; J.force = fs.force ? 1 : 0;
         J.needY = fs.needY ? 1 : 0; J.needX = fs.needX ? 1 : 0;
         J.rsY = fs.rsY; J.rsX = fs.rsX;
-        J.bC = bs.C; J.bcs = bs.cs; J.nchunk = bs.nchunk; J.groups = bs.groups; J.vpg = bs.vpg;
+        J.bC = bs.C; J.bcs = bs.cs; J.bpad = bs.pad; J.nchunk = bs.nchunk; J.groups = bs.groups; J.vpg = bs.vpg;
         J.fbp = bs.fbp ? 1 : 0;
         // forward
-        J.tr_gx = ceil_div(S.g.nx, 32);
+        J.tr_gx = ceil_div(S.g.nx + 2 * fs.pad, 32);
+        J.tr_xx = ceil_div(S.g.nx, 32);
         J.tr_gy = ceil_div(fs.cs, 32);
         DDLaunch c;
         c.kind = DDL_COPY;
-        add(fwd, c, j, (long)(J.needY + J.needX) * J.tr_gx * J.tr_gy * S.g.ny);
+        add(fwd, c, j, (long)J.needY * J.tr_gx * J.tr_gy * S.g.ny +
+                           (long)J.needX * J.tr_xx * J.tr_gy * (S.g.ny + 2 * fs.pad));
         DDLaunch f;
         f.fan = S.fan;
         f.ch = fs.CH;
@@ -2343,9 +2687,9 @@ void DDBatchPlan::Impl::layout() {
         } else {
             f.kind = DDL_FP;
             f.xc = fs.xc;
-            f.vpb = (fs.lseg == 0 && (tv == 2 || tv == 4)) ? tv : 1;
-            f.block = f.vpb > 1 ? 64 * f.vpb : 128;
-            J.fp_gx = f.vpb > 1 ? ceil_div(S.d.nu, 64) : ceil_div(S.d.nu, 128 >> fs.lseg);
+            f.vpb = fp_block_form(fs.lseg, tv);
+            f.block = f.vpb == 1 ? 128 : 64 * std::abs(f.vpb);
+            J.fp_gx = ceil_div(S.d.nu, f.vpb == 1 && fs.lseg == 0 ? 128 : 64);
             J.fp_gy = f.vpb > 1 ? ceil_div(S.nview, f.vpb) : S.nview;
             add(fwd, f, j, (long)J.fp_gx * J.fp_gy * fs.nchunk);
         }
@@ -2354,7 +2698,7 @@ void DDBatchPlan::Impl::layout() {
         DDLaunch z;
         z.kind = DDL_ZERO;
         add(bwd, z, j, (nimg + 1023) / 1024);
-        J.pr_gx = ceil_div(S.d.nu, 32);
+        J.pr_gx = ceil_div(S.d.nu + 2 * bs.pad, 32);
         J.pr_gy = ceil_div(bs.cs, 32);
         DDLaunch pr;
         pr.kind = DDL_PREP;

@@ -886,7 +886,7 @@ struct FBPView {
 // inlined.
 template <bool FAN>
 __device__ inline void fbp_view_point(float px, float py, float c, float s, float du, float off_u, float half,
-                                      float dso, float& pu, float& dist) {
+                                      float dso, bool narrow, float& pu, float& dist) {
 #pragma clang fp contract(off)
     const float rx = fmaf(px, c, py * s);
     const float ry = fmaf(py, c, -(px * s));
@@ -894,7 +894,7 @@ __device__ inline void fbp_view_point(float px, float py, float c, float s, floa
     dist = 1.f;
     if (FAN) {
         const float ys = dso + ry;
-        a = atanf(fast_div(rx, ys));
+        a = fan_atan(fast_div(rx, ys), narrow);
         dist = fast_div(dso * dso, fmaf(rx, rx, ys * ys));
     }
     pu = half - (fast_div(a, du) + off_u);
@@ -920,11 +920,12 @@ __global__ __launch_bounds__(256) void fan_fbp_bp_kernel(float* __restrict__ img
 #pragma unroll
     for (int j = 0; j < CH; j++) acc[j] = 0.f;
     const float half = (d.nu - 1.0f) / 2.0f;
+    const bool narrow = FAN && fan_narrow(g, dso);
     const size_t vstride = (size_t)d.nu * cs;
     for (int view = vbeg; view < vend; view++) {
         const FBPView V = views[view];
         float pu, dist;
-        fbp_view_point<FAN>(px, py, V.c, V.s, d.du, d.off_u, half, dso, pu, dist);
+        fbp_view_point<FAN>(px, py, V.c, V.s, d.du, d.off_u, half, dso, narrow, pu, dist);
         // InterpolateXY with truncation, cuda/cudaMath.cu:227-260
         if (pu < 0.f || pu >= (float)d.nu) continue;
         const int u0 = (int)pu;
@@ -982,13 +983,14 @@ __global__ __launch_bounds__(256) void fan_fbp_bp_split_kernel(float* __restrict
 #pragma unroll
     for (int j = 0; j < 4 * NQ; j++) acc[j] = 0.f;
     const float half = (d.nu - 1.0f) / 2.0f;
+    const bool narrow = FAN && fan_narrow(g, dso);
     const size_t vstride = (size_t)d.nu * cs;
     const unsigned lane_b = 16u * sub;   // the lane's first float of a cell, in bytes
     for (int v0 = vbeg; v0 < vend; v0 += LPC) {
         float mpu = -1.f, mdist = 0.f;
         if (v0 + sub < vend) {
             const FBPView V = views[v0 + sub];
-            fbp_view_point<FAN>(px, py, V.c, V.s, d.du, d.off_u, half, dso, mpu, mdist);
+            fbp_view_point<FAN>(px, py, V.c, V.s, d.du, d.off_u, half, dso, narrow, mpu, mdist);
         }
 #pragma unroll
         for (int t = 0; t < LPC; t++) {
@@ -1082,6 +1084,7 @@ __global__ __launch_bounds__(256) void fan_fbp_bp_stage_kernel(float* __restrict
 #pragma unroll
     for (int j = 0; j < 4 * NQ; j++) acc[j] = 0.f;
     const float half = (d.nu - 1.0f) / 2.0f;
+    const bool narrow = FAN && fan_narrow(g, dso);
     const size_t vstride = (size_t)d.nu * cs;
     int fo[NQ];                             // float4 index within a cell of accumulator k
 #pragma unroll
@@ -1099,7 +1102,7 @@ __global__ __launch_bounds__(256) void fan_fbp_bp_stage_kernel(float* __restrict
         float mpu = -1.f, mdist = 0.f;
         int lo = 1 << 30, hi = -1;   // empty
         if (v0 + sub < vend) {
-            fbp_view_point<FAN>(px, py, vc, vs, d.du, d.off_u, half, dso, mpu, mdist);
+            fbp_view_point<FAN>(px, py, vc, vs, d.du, d.off_u, half, dso, narrow, mpu, mdist);
             if (valid && mpu >= 0.f && mpu < (float)d.nu) {
                 lo = (int)mpu;
                 hi = min(lo + 1, d.nu - 1);

@@ -41,7 +41,7 @@ std::map<std::string, int> g_tune = {
     {"cone_plan_persistent", 0},   // cone plans: 1 persistent blocks with work counters, 2 one block per tile
     {"dd_batch_persistent", 0},    // DD batch plans: 1 persistent blocks with work counters, 2 one block per tile (default)
     {"dd_batch_streams", 0},       // DD batch plans: streams the kernel classes of a direction run on (1 to 4; default 4)
-    {"dd_fp_mode", 0},       // DD FP: 1 direct (default), 2 LDS-staged rows where the footprint fits
+    {"dd_fp_mode", 0},       // DD FP: 0 window form up to 4 channels, 1 pixel-by-pixel walk, 2 LDS-staged rows where the footprint fits
     {"dd_fp_extra_channel", 0},  // DD FP direct kernel: 1 keeps the next chunk's channel with one chunk too
     {"dd_fp_pixel_stride", 0},   // DD FP direct kernel, one channel chunk: floats per pixel of the channel-last copy
     {"dd_fp_views_per_block", 0},  // DD FP direct kernel, one row segment: views per block (1, 2, 4; default 4)
@@ -49,7 +49,7 @@ std::map<std::string, int> g_tune = {
     {"dd_bp_lanes_per_pixel", 0},  // DD BP (pixel driven): lanes per pixel (1 = whole channel vector per lane; 2, 4; default 4 at 32 channels, else 2)
     {"fbp_bp_lanes_per_pixel", 0}, // fan FBP / parallel pixel BP: lanes per pixel (1 = whole channel vector per lane; 2, 4; default 4, 2 at 8 channels)
     {"fbp_bp_stage", 0},     // fan FBP / parallel pixel BP, split form: cells staged in LDS per wavefront: 1 always, 2 never (default: at 32 channels with 4 lanes per pixel)
-    {"dd_fp_segments", 0},   // DD FP direct kernel: row segments per column (1, 2; default by wave count)
+    {"dd_fp_segments", 0},   // DD FP direct kernel: row segments per column (1, 2, or 3 / 4 for 4 / 8 segments up to 8 channels; default by wave count)
     {"tv_mode", 0},          // TV prior: 1 z-marching tile kernels (default), 2 one lane per voxel
     {"ramp_mode", 0},        // ramp filter: 0 FFT convolution where 2nu-1 <= 4096 (default), 1 direct, 2 generic FFT kernel
     {"bp_view_groups", 0},   // view groups of the pixel-driven DD / FBP backprojections (default: enough for 1024 blocks)

@@ -538,3 +538,48 @@ def test_parallel_pixel_bp(oracle, variant):
     y = np.random.default_rng(5).uniform(size=[img.shape[0], len(ang), g.nv, g.nu]).astype(np.float32)
     bp = parallel.pixel_driven_bp(_proj(g), y, ang)
     assert rel_l2(bp, oracle.par_pixel_bp(g, y, ang)) < TOL
+
+
+@pytest.mark.parametrize('nz', [1, 2, 3, 4])
+@pytest.mark.parametrize('case', ['fine', 'coarse', 'wide', 'beside', 'steep_fan', 'parallel', 'parallel_wide'])
+def test_dd_window_form(oracle, tuning, case, nz):
+    """The window form of the DD projectors (up to 4 slices) against the oracle
+    and, for the FP, against the pixel-by-pixel walk (dd_fp_mode 1): footprints
+    under 1, under 2 and over 2 pixels (cells) wide, an image most columns pass
+    on one side, a fan wider than the polynomial arctangent's range, row counts
+    with remainders and row segments.  A pixel that is not finite spoils the
+    same rays in both forms."""
+    fan_beam = not case.startswith('parallel')
+    kw = dict(nx=101, ny=75, nz=nz, dx=1.0, dy=1.0, dz=1.0, cx=1.3, cy=-0.6, nu=97, nv=nz, du=1.37, dv=1.0, off_u=0.31)
+    if fan_beam:
+        kw.update(dsd=400.0, dso=240.0, du=2.0)
+    if case == 'fine':
+        kw.update(du=0.9, nu=200)
+    if case == 'wide':
+        kw.update(du=7.0, nu=40)
+    if case == 'parallel_wide':
+        kw.update(du=0.3, nu=300)
+    if case == 'beside':
+        kw.update(nx=40, cx=30.0, cy=25.0)
+    if case == 'steep_fan':
+        kw.update(dsd=160.0, dso=80.0, du=3.0, nu=120)
+    g = Geo(**kw)
+    ang = (np.arange(29) * (2 if fan_beam else 1) * np.pi / 29 + 0.013).astype(np.float32)
+    rng = np.random.default_rng(12)
+    img = rng.uniform(size=[1, nz, g.ny, g.nx]).astype(np.float32)
+    m = fan if fan_beam else parallel
+    fp_ref, bp_ref = (oracle.dd_fan_fp, oracle.dd_fan_bp) if fan_beam else (oracle.dd_par_fp, oracle.dd_par_bp)
+    p = _proj(g)
+    a = m.distance_driven_fp(p, img, ang)
+    y = rng.uniform(size=a.shape).astype(np.float32)
+    errs = [rel_l2(a, fp_ref(g, img, ang))]
+    for is_fbp in (False, True):
+        errs.append(rel_l2(m.distance_driven_bp(p, y, ang, is_fbp=is_fbp), bp_ref(g, y, ang, is_fbp=is_fbp)))
+    img[0, nz - 1, 30, 17] = np.nan
+    img[0, 0, 50, 33] = np.inf
+    bad = m.distance_driven_fp(p, img, ang)
+    tuning('dd_fp_mode', 1)
+    walk = m.distance_driven_fp(p, img, ang)
+    print('dd window', case, nz, errs)
+    assert max(errs) < TOL
+    assert np.array_equal(np.isnan(bad), np.isnan(walk)) and np.array_equal(np.isinf(bad), np.isinf(walk))
