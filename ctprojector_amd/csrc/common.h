@@ -65,6 +65,13 @@ __device__ inline float min_f(float a, float b) { return med3_f(a, b, -3.0e38f);
 __device__ inline float max_f(float a, float b) { return med3_f(a, b, 3.0e38f); }
 
 #ifdef __HIPCC__
+// The legacy product: 0 * x = 0 for every x, also where x is not finite.
+__device__ inline float mul_legacy(float a, float b) {
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
 // atan(t) for |t| <= 0.7 ('narrow', uniform across the wavefront), else through
 // the library: t + t z P(z), z = t^2, with P the degree-6 Chebyshev
 // interpolant of (atan(t)/t - 1)/z on [0, 0.5] (within 1 ulp; 9 instructions

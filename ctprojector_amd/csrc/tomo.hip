@@ -23,6 +23,7 @@
 #include "ops.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace ctp {
 
@@ -45,6 +46,90 @@ __device__ inline float box_xy(const float* __restrict__ p, float x1, float y1, 
 }
 
 __device__ inline float3 ld3t(const float* p, int i) { return make_float3(p[3 * i], p[3 * i + 1], p[3 * i + 2]); }
+
+// Interval [a, b] (clamped to [0, n], n >= K) over K consecutive cells from
+// cell e on: the overlaps w.  e is moved inwards at the row's end, so that the
+// K cells exist.
+template <int K>
+struct Span {
+    float w[K];
+    int e;
+    __device__ inline Span(float a, float b, int n) {
+        const float f = min_f(floorf(a), (float)(n - K));
+        e = (int)f;
+        float edge = med3_f(f, a, b);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const float next = med3_f(f + (float)(k + 1), a, b);
+            w[k] = next - edge;
+            edge = next;
+        }
+    }
+};
+
+// (Window form of the boxes: the loops of box_xy with their clamps, divisions
+// and dependent loads took 122 us forward and 150 us backward at 256^2 x 48
+// voxels, 9 views of 256^2 cells; the call now takes 138 instead of 300 us.
+// Cells a box does not meet weigh 0 by the legacy product, whatever they hold.)
+// The average of a plane (nx x ny cells) over the box [x1, x2] x [y1, y2], of
+// which at most K cells per axis are met: cells loaded ahead of their use.
+template <int K>
+struct BoxCells {
+    float q[K][K], wx[K], wy[K], inv;
+    __device__ inline void load(const float* __restrict__ p, int nx, int ny, float x1, float x2, float y1, float y2) {
+        typedef float vec __attribute__((ext_vector_type(K), aligned(4)));
+        inv = __builtin_amdgcn_rcpf((x2 - x1) * (y2 - y1));
+        const Span<K> x(med_clamp(x1, 0.f, (float)nx), med_clamp(x2, 0.f, (float)nx), nx);
+        const Span<K> y(med_clamp(y1, 0.f, (float)ny), med_clamp(y2, 0.f, (float)ny), ny);
+        const unsigned off = (unsigned)(y.e * nx + x.e);
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            wx[j] = x.w[j];
+            wy[j] = y.w[j];
+            const vec v = *reinterpret_cast<const vec*>(p + off + (unsigned)(j * nx));
+#pragma unroll
+            for (int i = 0; i < K; i++) q[j][i] = v[i];
+        }
+    }
+    __device__ inline float sum() const {
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            float r = mul_legacy(wx[0], q[j][0]);
+#pragma unroll
+            for (int i = 1; i < K; i++) r += mul_legacy(wx[i], q[j][i]);
+            const float t = mul_legacy(wy[j], r);
+            s = j == 0 ? t : s + t;
+        }
+        return s;
+    }
+};
+
+// FP planes of a lane in the window form: K cells per axis, two planes' loads
+// in flight.
+template <int K>
+__device__ inline float tomo_fp_planes(const float* __restrict__ img, const Grid& g, float3 s, float rx1, float rx2,
+                                       float ry1, float ry2) {
+    const size_t npl = (size_t)g.nx * g.ny;
+    float val = 0.f;
+    auto planes = [&](int iz, auto count) {
+        constexpr int N = decltype(count)::value;
+        BoxCells<K> B[N];
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const float h = (float)(iz + u) - s.z;
+            const float a1 = fmaf(rx1, h, s.x), a2 = fmaf(rx2, h, s.x);
+            const float b1 = fmaf(ry1, h, s.y), b2 = fmaf(ry2, h, s.y);
+            B[u].load(img + (size_t)(iz + u) * npl, g.nx, g.ny, a1, a2, b1, b2);
+        }
+#pragma unroll
+        for (int u = 0; u < N; u++) val = fmaf(B[u].sum(), B[u].inv, val);
+    };
+    int iz = 0;
+    for (; iz + 4 <= g.nz; iz += 4) planes(iz, std::integral_constant<int, 4>{});
+    for (; iz < g.nz; iz++) planes(iz, std::integral_constant<int, 1>{});
+    return val;
+}
 
 __global__ __launch_bounds__(256) void tomo_fp_kernel(float* __restrict__ prj, const float* __restrict__ img,
                                                       const float* __restrict__ pdc, const float* __restrict__ psrc,
@@ -71,14 +156,30 @@ __global__ __launch_bounds__(256) void tomo_fp_kernel(float* __restrict__ prj, c
     if (y1.y > y2.y) { const float3 t = y1; y1 = y2; y2 = t; }
     const float rx1 = (x1.x - s.x) / (x1.z - s.z), rx2 = (x2.x - s.x) / (x2.z - s.z);
     const float ry1 = (y1.y - s.y) / (y1.z - s.z), ry2 = (y2.y - s.y) / (y2.z - s.z);
+    // the boxes' sides are linear in the plane: the end planes' bound them
+    float side = 0.f, least = 3.0e38f;
+    for (int k = 0; k < 2; k++) {
+        const float h = (k == 0 ? 0.f : (float)(g.nz - 1)) - s.z;
+        const float w = fmaf(rx2, h, s.x) - fmaf(rx1, h, s.x), v = fmaf(ry2, h, s.y) - fmaf(ry1, h, s.y);
+        side = fmaxf(side, fmaxf(w, v));
+        least = fminf(least, fminf(w, v));
+    }
+    // (sides of no or negative length, a source within the volume's planes, stay with the loops)
+    const int cells = g.nx < 3 || g.ny < 3 || __any(!(least > 1e-6f)) ? 0
+                      : !__any(!(side < 0.999f))                    ? 2
+                      : !__any(!(side < 1.999f))                    ? 3
+                                                                    : 0;   // uniform
     float val = 0.f;
     const size_t npl = (size_t)g.nx * g.ny;
-    for (int iz = 0; iz < g.nz; iz++) {
-        const float h = (float)iz - s.z;
-        const float a1 = s.x + rx1 * h, a2 = s.x + rx2 * h;
-        const float b1 = s.y + ry1 * h, b2 = s.y + ry2 * h;
-        val += box_xy(img + iz * npl, a1, b1, a2, b2, g.nx, g.ny) / ((a2 - a1) * (b2 - b1));
-    }
+    if (cells == 2) val = tomo_fp_planes<2>(img, g, s, rx1, rx2, ry1, ry2);
+    else if (cells == 3) val = tomo_fp_planes<3>(img, g, s, rx1, rx2, ry1, ry2);
+    else
+        for (int iz = 0; iz < g.nz; iz++) {
+            const float h = (float)iz - s.z;
+            const float a1 = fmaf(rx1, h, s.x), a2 = fmaf(rx2, h, s.x);
+            const float b1 = fmaf(ry1, h, s.y), b2 = fmaf(ry2, h, s.y);
+            val += box_xy(img + iz * npl, a1, b1, a2, b2, g.nx, g.ny) / ((a2 - a1) * (b2 - b1));
+        }
     const float3 D = make_float3(C.x + u, C.y + v, C.z);
     val *= g.dz / fabsf(S.z - D.z) *
            sqrtf((S.z - D.z) * (S.z - D.z) + (S.y - D.y) * (S.y - D.y) + (S.x - D.x) * (S.x - D.x));
@@ -128,17 +229,46 @@ __global__ __launch_bounds__(256) void tomo_bp_kernel(float* __restrict__ img, c
     const float z = ((float)iz - (g.nz - 1) / 2.0f) * g.dz + g.cz;
     const float ou = d.off_u + (d.nu - 1) / 2.0f, ov = d.off_v + (d.nv - 1) / 2.0f;
     const size_t nuv = (size_t)d.nu * d.nv;
+    const float rdu = 1.f / d.du, rdv = 1.f / d.dv;
     float val = 0.f;
-    for (int view = 0; view < nview; view++) {
-        const float3 S = ld3t(psrc, view), C = ld3t(pdc, view);
-        // ProjectConeToDetCart, cuda/distanceDriven3DUtils.cu:45-56
-        const float r = (C.z - S.z) / (z - S.z);
-        const float u1 = (S.x - C.x + r * (x - g.dx / 2 - S.x)) / d.du + ou;
-        const float u2 = (S.x - C.x + r * (x + g.dx / 2 - S.x)) / d.du + ou;
-        const float v1 = (S.y - C.y + r * (y - g.dy / 2 - S.y)) / d.dv + ov;
-        const float v2 = (S.y - C.y + r * (y + g.dy / 2 - S.y)) / d.dv + ov;
-        val += box_xy(w + view * nuv, u1, v1, u2, v2, d.nu, d.nv) / ((u2 - u1) * (v2 - v1));
-    }
+    // shadow of the voxel on view's detector, ProjectConeToDetCart, cuda/distanceDriven3DUtils.cu:45-56
+    // (the magnification, its divisions and the offsets are the same in every lane)
+    auto shadow = [&](int view, float& u1, float& u2, float& v1, float& v2) {
+        const float Sx = const_load(psrc, 3L * view), Sy = const_load(psrc, 3L * view + 1);
+        const float Sz = const_load(psrc, 3L * view + 2), Cz = const_load(pdc, 3L * view + 2);
+        const float r = (Cz - Sz) / (z - Sz);
+        const float tx = Sx - const_load(pdc, 3L * view), ty = Sy - const_load(pdc, 3L * view + 1);
+        u1 = fmaf(fmaf(r, x - g.dx / 2 - Sx, tx), rdu, ou);
+        u2 = fmaf(fmaf(r, x + g.dx / 2 - Sx, tx), rdu, ou);
+        v1 = fmaf(fmaf(r, y - g.dy / 2 - Sy, ty), rdv, ov);
+        v2 = fmaf(fmaf(r, y + g.dy / 2 - Sy, ty), rdv, ov);
+    };
+    auto batch = [&](int view, auto count) {
+        constexpr int N = decltype(count)::value;
+        float u1[N], u2[N], v1[N], v2[N];
+        float side = 0.f, least = 3.0e38f;
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            shadow(view + k, u1[k], u2[k], v1[k], v2[k]);
+            side = fmaxf(side, fmaxf(u2[k] - u1[k], v2[k] - v1[k]));
+            least = fminf(least, fminf(u2[k] - u1[k], v2[k] - v1[k]));
+        }
+        if (d.nu >= 3 && d.nv >= 3 && !__any(!(side < 1.999f) || !(least > 1e-6f))) {   // uniform
+            BoxCells<3> B[N];
+#pragma unroll
+            for (int k = 0; k < N; k++) B[k].load(w + (view + k) * nuv, d.nu, d.nv, u1[k], u2[k], v1[k], v2[k]);
+#pragma unroll
+            for (int k = 0; k < N; k++) val = fmaf(B[k].sum(), B[k].inv, val);
+        } else {
+#pragma unroll
+            for (int k = 0; k < N; k++)
+                val += box_xy(w + (view + k) * nuv, u1[k], v1[k], u2[k], v2[k], d.nu, d.nv) /
+                       ((u2[k] - u1[k]) * (v2[k] - v1[k]));
+        }
+    };
+    int view = 0;
+    for (; view + 2 <= nview; view += 2) batch(view, std::integral_constant<int, 2>{});
+    for (; view < nview; view++) batch(view, std::integral_constant<int, 1>{});
     img[((size_t)iz * g.ny + iy) * g.nx + ix] = val;
 }
 

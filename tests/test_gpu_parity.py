@@ -583,3 +583,39 @@ def test_dd_window_form(oracle, tuning, case, nz):
     print('dd window', case, nz, errs)
     assert max(errs) < TOL
     assert np.array_equal(np.isnan(bad), np.isnan(walk)) and np.array_equal(np.isinf(bad), np.isinf(walk))
+
+
+@pytest.mark.parametrize('case', ['fine', 'coarse', 'wide', 'flat', 'truncated'])
+def test_tomo_window_form(oracle, case):
+    """The window form of the tomosynthesis projector against the oracle: boxes
+    under 1, under 2 and over 2 cells, planes of 2 rows (no window), plane and
+    view counts with remainders, boxes past the edges; a cell that is not
+    finite reaches only the rays and voxels whose boxes meet it."""
+    kw = dict(nx=37, ny=29, nz=11, dx=1.0, dy=1.0, dz=1.0, cz=20.0, nu=43, nv=39, du=1.03, dv=0.97, off_u=0.2)
+    if case == 'fine':
+        kw.update(du=0.7, dv=0.6, nu=61, nv=57)
+    if case == 'wide':
+        kw.update(du=2.9, dv=2.7, nu=15, nv=13)
+    if case == 'flat':
+        kw.update(ny=2, nv=7)
+    if case == 'truncated':
+        kw.update(nu=20, nv=11, cx=6.0)
+    g = Geo(**kw)
+    t = np.linspace(-0.4, 0.4, 5)
+    src = np.stack([300 * np.sin(t), 5 * np.ones_like(t), 300 * np.cos(t) + 20], 1).astype(np.float32)
+    dc = np.stack([0 * t, 0 * t, 0 * t - 10], 1).astype(np.float32)
+    rng = np.random.default_rng(9)
+    p = _proj(g)
+    img = rng.uniform(size=[1, g.nz, g.ny, g.nx]).astype(np.float32)
+    y = rng.uniform(size=[1, 5, g.nv, g.nu]).astype(np.float32)
+    fp, ref = tomo.distance_driven_fp(p, img, dc, src), oracle.dd_tomo_fp(g, img, dc, src)
+    bp, refb = tomo.distance_driven_bp(p, y, dc, src), oracle.dd_tomo_bp(g, y, dc, src)
+    e = rel_l2(fp, ref), rel_l2(bp, refb)
+    print('tomo window', case, e)
+    assert max(e) < TOL
+    unit, lit = np.zeros_like(img), img.copy()
+    unit[0, 4, 1, 20], lit[0, 4, 1, 20] = 1.0, np.nan
+    met = oracle.dd_tomo_fp(g, unit, dc, src) > 1e-4
+    bad = np.isnan(tomo.distance_driven_fp(p, lit, dc, src))
+    # (the lit voxel lies beside the truncated panel: no ray meets it)
+    assert met.any() == (case != 'truncated') and bad[met].all() and bad.sum() <= met.sum() + 2
