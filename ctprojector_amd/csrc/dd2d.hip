@@ -270,13 +270,6 @@ __device__ inline void fp_trace_rows(float* acc, const float* __restrict__ img, 
 // -> 494.
 constexpr int kPad = 4;
 
-// 0 * x = 0 for every x
-__device__ inline float mul_legacy(float a, float b) {
-    float r;
-    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
 // K pixels of one row (or of one view's detector row), rows[0] the first pad
 // pixel: weights w[K] (w[0] first) of the footprint between lo and hi, and the
 // channel vectors.
@@ -294,7 +287,7 @@ struct Window {
             edge = next;
         }
         // byte offset from the row's first pad; footprints beyond the row read pads
-        const unsigned off = (unsigned)__mul24((int)med_clamp(fl, -(float)kPad, nf), 4 * CH) + 4u * kPad * CH;
+        const unsigned off = (unsigned)((int)med_clamp(fl, -(float)kPad, nf) + kPad) * (4u * CH);
         const char* __restrict__ rb = reinterpret_cast<const char*>(row);
         if constexpr (CH <= 2) {
             typedef float vec __attribute__((ext_vector_type(K * CH), aligned(4 * CH)));
@@ -1067,7 +1060,7 @@ static DDFPSetup dd_fp_setup(const std::vector<DDView>& views, int B, const Grid
     // keeps the pixel-by-pixel walk); at 8 the third pixel's 32 bytes cost more
     // than the arithmetic saves (512^2 / 984 views, fan: walk 1.28 ms, window 1.64)
     if (!split && !s.xc && !s.use_lds && CH <= 4 && s.cs == CH && tuning_get("dd_fp_mode", 0) == 0 &&
-        (long)(std::max(g.nx, g.ny) + 2 * kPad) * CH < (1 << 21))
+        std::max(g.nx, g.ny) + 2 * kPad <= 65535)   // (rows of the x-major copy are its launch's third dimension)
         s.pad = kPad;
     s.rsY = (long)(g.nx + 2 * s.pad) * s.cs;
     s.rsX = (long)(g.ny + 2 * s.pad) * s.cs;
