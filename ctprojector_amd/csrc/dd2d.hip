@@ -955,7 +955,8 @@ struct DDFPSetup {
 // lpc_req > 0: lanes per column requested instead of the tuning key, reduced
 // to what the chunk allows (CH / 4; 1 = the one-lane kernel).
 static DDFPSetup dd_fp_setup(const std::vector<DDView>& views, int B, const Grid& g, const Det& d, int nview,
-                             float dsd, float dso, int type, bool fan, bool allow_lds = true, int lpc_req = 0) {
+                             float dsd, float dso, int type, bool fan, bool allow_lds = true, int lpc_req = 0,
+                             bool allow_window = true) {
     const bool branchless = (type & DD_BRANCHLESS) != 0;
     DDFPSetup s;
     s.C = B * g.nz;
@@ -1059,7 +1060,7 @@ static DDFPSetup dd_fp_setup(const std::vector<DDView>& views, int B, const Grid
     // up to 4 channels the one-lane kernel runs the window form (dd_fp_mode 1
     // keeps the pixel-by-pixel walk); at 8 the third pixel's 32 bytes cost more
     // than the arithmetic saves (512^2 / 984 views, fan: walk 1.28 ms, window 1.64)
-    if (!split && !s.xc && !s.use_lds && CH <= 4 && s.cs == CH && tuning_get("dd_fp_mode", 0) == 0 &&
+    if (allow_window && !split && !s.xc && !s.use_lds && CH <= 4 && s.cs == CH && tuning_get("dd_fp_mode", 0) == 0 &&
         std::max(g.nx, g.ny) + 2 * kPad <= 65535)   // (rows of the x-major copy are its launch's third dimension)
         s.pad = kPad;
     s.rsY = (long)(g.nx + 2 * s.pad) * s.cs;
@@ -1250,8 +1251,12 @@ static char* noalloc_scratch() {
 void dd2d_fp_noalloc(float* prj, const float* img, const float* deg_host, int B, const Grid& g, const Det& d,
                      int nview, float dsd, float dso, int type, bool fan, hipStream_t stream) {
     const std::vector<DDView> views = dd_views_for(deg_host, nview, g, type);
-    const DDFPSetup s = dd_fp_setup(views, B, g, d, nview, dsd, dso, type, fan);
-    const size_t bytes = dd_fp_scratch_bytes(s, g, nview);
+    DDFPSetup s = dd_fp_setup(views, B, g, d, nview, dsd, dso, type, fan);
+    size_t bytes = dd_fp_scratch_bytes(s, g, nview);
+    if (bytes > kDDFPNoAllocScratchBytes && s.pad > 0) {   // the walk needs no pads in the copies
+        s = dd_fp_setup(views, B, g, d, nview, dsd, dso, type, fan, true, 0, false);
+        bytes = dd_fp_scratch_bytes(s, g, nview);
+    }
     if (bytes > kDDFPNoAllocScratchBytes)
         fail("the allocation-free forward projection needs " + std::to_string(bytes) +
              " bytes of scratch, more than its fixed " + std::to_string(kDDFPNoAllocScratchBytes) +

@@ -72,3 +72,27 @@ def test_no_alloc_refuses_oversized_call():
     assert lib.ctpDistanceDrivenFanProjectionNoAlloc(*_args(b, img2, ang2, p2)) == 0
     torch.cuda.synchronize()
     assert torch.equal(a, b)
+
+
+def test_no_alloc_walks_where_padded_copies_do_not_fit():
+    """Four slices of 1616^2: the two channel-last copies fit the array only
+    without the zero columns of the window form, so the call takes the
+    pixel-by-pixel walk; bit for bit the allocating entry point's walk."""
+    import torch
+    from ctprojector_amd import _lib
+    lib = _lib.module()
+    dev = torch.device('cuda', 0)
+    n = 1616
+    assert 2 * 16 * n * n < SCRATCH_BYTES < 2 * 16 * n * (n + 8)
+    img, ang, p, oshape = _case(torch, 4, 1, 4, n, 6, 300, 0)
+    a = torch.zeros(oshape, device=dev)
+    b = torch.full(oshape, 7.0, device=dev)
+    _lib.set_tuning('dd_fp_mode', 1)
+    try:
+        assert lib.cupyDistanceDrivenFanProjection(*_args(a, img, ang, p)) == 0
+    finally:
+        _lib.set_tuning('dd_fp_mode', 0)
+    assert lib.ctpDistanceDrivenFanProjectionNoAlloc(*_args(b, img, ang, p)) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(a, b), float((a - b).abs().max())
+    assert float(a.abs().max()) > 0
