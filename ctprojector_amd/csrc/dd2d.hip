@@ -1915,8 +1915,12 @@ void dd2d_bp(float* img, const float* prj, const float* deg_host, int B, const G
 // recomputed from the same FP32 line parameters the forward projector uses.
 // Candidates whose weight is not positive add 0 times their channels, so a
 // non-finite detector value also reaches the pixels next to its footprint.
+// Bound by the L1's data path: a candidate is its record and its channels.  In
+// the fan beam half of the record is the source, read once per view and trace
+// instead (8 slices of 256^2, 492 views, 444 columns: 203 -> 146 us).
 struct FPTrace {           // one trace of a (view, column): edge lines r * (t - o) + b and the norm
-    float r1, o1, b1, r2, o2, b2, norm, pad;
+    float r1, r2, norm, pad;
+    float o1, b1, o2, b2;  // the source in the fan beam: the same for every column of a view
 };
 struct FPLine {            // per (view, column): trace along y (x of row t), trace along x (y of column t)
     FPTrace tr[2];         // 32-byte aligned records: a candidate's trace is two 16-byte loads
@@ -1932,11 +1936,11 @@ __global__ __launch_bounds__(256) void dd_fp_lines_kernel(FPLine* __restrict__ l
     const float a = fp_cell_edges<FAN>(iu, V, g, d, dsd, dso, s1, s2, d1, d2);
     FPLine L{};
     if (V.flags & 1)
-        L.tr[0] = FPTrace{(d1.x - s1.x) / (d1.y - s1.y), s1.y, s1.x, (d2.x - s2.x) / (d2.y - s2.y), s2.y, s2.x,
-                          V.wx * g.dy / fabsf(cosf(V.deg - a)), 0.f};
+        L.tr[0] = FPTrace{(d1.x - s1.x) / (d1.y - s1.y), (d2.x - s2.x) / (d2.y - s2.y),
+                          V.wx * g.dy / fabsf(cosf(V.deg - a)), 0.f, s1.y, s1.x, s2.y, s2.x};
     if (V.flags & 2)
-        L.tr[1] = FPTrace{(d1.y - s1.y) / (d1.x - s1.x), s1.x, s1.y, (d2.y - s2.y) / (d2.x - s2.x), s2.x, s2.y,
-                          (1.f - V.wx) * g.dx / fabsf(sinf(V.deg - a)), 0.f};
+        L.tr[1] = FPTrace{(d1.y - s1.y) / (d1.x - s1.x), (d2.y - s2.y) / (d2.x - s2.x),
+                          (1.f - V.wx) * g.dx / fabsf(sinf(V.deg - a)), 0.f, s1.x, s1.y, s2.x, s2.y};
     lines[(size_t)view * d.nu + iu] = L;
 }
 
@@ -2019,13 +2023,15 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
             const float t = tr == 0 ? (float)iy + 0.5f : (float)ix + 0.5f;
             const int n = tr == 0 ? g.nx : g.ny;
             const float lo = tr == 0 ? (float)ix : (float)iy;
+            // (fan beam: the trace's origin is the source, one for all columns; half a record per candidate)
+            const float4 org = const_load(reinterpret_cast<const float4*>(&Lv[0].tr[tr]), 1);
             for (int k = k0; k <= k1; k++) {
                 // the candidate's trace record and its channels load together
                 // (one memory round trip per candidate; taking candidates in
                 // pairs measured slower); a candidate whose weight is not
                 // positive adds 0 times its channels
                 const float4* __restrict__ lp = reinterpret_cast<const float4*>(&Lv[k].tr[tr]);
-                const float4 l0 = lp[0], l1 = lp[1];   // r1 o1 b1 r2 | o2 b2 norm -
+                const float4 l0 = lp[0], l1 = FAN ? org : lp[1];   // r1 r2 norm - | o1 b1 o2 b2
                 float q[CH];
                 const float* __restrict__ gp = Gv + (size_t)k * cs;
                 if constexpr (CH % 4 == 0) {
@@ -2038,11 +2044,11 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
 #pragma unroll
                     for (int j = 0; j < CH; j++) q[j] = gp[j];
                 }
-                const float x1 = fmaf(l0.x, t - l0.y, l0.z), x2 = fmaf(l0.w, t - l1.x, l1.y);
+                const float x1 = fmaf(l0.x, t - l1.x, l1.y), x2 = fmaf(l0.y, t - l1.z, l1.w);
                 // the forward projector's IntegralBoxX weight of this pixel (dd_line)
                 const float xl = min_f(x1, x2), xh = max_f(x1, x2);
                 const float a = med_clamp(xl, 0.f, (float)n), b = med_clamp(xh, 0.f, (float)n);
-                const float wt = (fminf(b, lo + 1.f) - fmaxf(a, lo)) * fast_div(l1.z, xh - xl);
+                const float wt = (fminf(b, lo + 1.f) - fmaxf(a, lo)) * fast_div(l0.z, xh - xl);
                 const float w = (b > a && wt > 0.f) ? wt : 0.f;
 #pragma unroll
                 for (int j = 0; j < CH; j++) acc[j] = fmaf(w, q[j], acc[j]);
