@@ -1132,8 +1132,13 @@ __global__ __launch_bounds__(256) void siddon_bp_coltable_kernel(float* __restri
 }
 
 // The rays left at weight 0 by siddon_bp_coltable_kernel: FP64 weight into
-// their dup entries, and the exact scatter of exception rays.  Grid: (row
-// groups of 8, views); blocks of rows without a flag return at once.
+// their dup entries, and the exact scatter of exception rays.  Block (part,
+// view) takes every gridDim.x-th row of its view and reads 256 row flags at a
+// time: hardly any row is flagged, so a block's time is mostly that one load's
+// latency (a block per 8 rows, reading its flags one by one, took 70 us at
+// 256^3 / 720 views).  Where rows are flagged their rays cost far more than the
+// flags, so few views are split into more parts (128^3 and 60 views with flagged
+// rows: 70 us, one exact ray's time; 190 us with one block per view).
 __global__ __launch_bounds__(256) void siddon_bp_colpatch_kernel(float* __restrict__ wtab, float* __restrict__ img,
                                                                  const int* __restrict__ rowirr,
                                                                  const float* __restrict__ prj,
@@ -1145,16 +1150,24 @@ __global__ __launch_bounds__(256) void siddon_bp_colpatch_kernel(float* __restri
                                                                  const float* __restrict__ psrc, Grid g, Det d,
                                                                  int dup) {
     const int view = blockIdx.y;
-    for (int r = 0; r < kTabRows; r++) {
-        const int iv = blockIdx.x * kTabRows + r;
-        if (iv >= d.nv) return;
-        if (rowirr[(long)view * d.nv + iv] == 0) continue;
-        for (int iu = threadIdx.x; iu < d.nu; iu += 256) {
-            const long i = ((long)view * d.nv + iv) * d.nu + iu;
-            if (coltable_fast(i, iu, iv, view, prj, colw, roww, psrc, g, d) >= 0.f) continue;
-            const float w = coltable_exact(i, iu, iv, view, true, img, prj, pdc, pdu, pdv, psrc, g, d);
-            for (int jv = 0; jv < dup && jv <= iv; jv++) wtab[(i - (long)jv * d.nu) * dup + jv] = w;
+    __shared__ int list[256], count;
+    for (int base = blockIdx.x; base < d.nv; base += 256 * gridDim.x) {
+        if (threadIdx.x == 0) count = 0;
+        __syncthreads();
+        const int row = base + threadIdx.x * gridDim.x;
+        if (row < d.nv && rowirr[(long)view * d.nv + row] != 0) list[atomicAdd(&count, 1)] = row;
+        __syncthreads();
+        const int n = count;
+        for (int r = 0; r < n; r++) {
+            const int iv = list[r];
+            for (int iu = threadIdx.x; iu < d.nu; iu += 256) {
+                const long i = ((long)view * d.nv + iv) * d.nu + iu;
+                if (coltable_fast(i, iu, iv, view, prj, colw, roww, psrc, g, d) >= 0.f) continue;
+                const float w = coltable_exact(i, iu, iv, view, true, img, prj, pdc, pdu, pdv, psrc, g, d);
+                for (int jv = 0; jv < dup && jv <= iv; jv++) wtab[(i - (long)jv * d.nu) * dup + jv] = w;
+            }
         }
+        __syncthreads();   // the list is read before the next stretch's replaces it
     }
 }
 
@@ -1929,6 +1942,7 @@ static void siddon_cone_bp_grid(float* img, const float* prj, const ConeGeomDev&
                 utab, vtab, qtab, colw, roww, dviews, geo.det_center, geo.det_u, geo.det_v, geo.src, g, d, nview);
             CTP_LAUNCH_CHECK();
         }
+        const int patch_parts = std::min(std::max(8192 / nview, 1), d.nv);
         for (int b = 0; b < B;) {
             const int nb = B - b >= 4 && nbmax >= 4 ? 4 : (B - b >= 2 && nbmax >= 2 ? 2 : 1);
             WTabs wt{{nullptr, nullptr, nullptr, nullptr}};
@@ -1948,7 +1962,7 @@ static void siddon_cone_bp_grid(float* img, const float* prj, const ConeGeomDev&
                     default: siddon_bp_coltable_kernel<4><<<tg, 256, 0, stream>>>(wk, rowirr, pk, colw, roww, geo.src, g, d); break;
                 }
                 CTP_LAUNCH_CHECK();
-                siddon_bp_colpatch_kernel<<<dim3(ceil_div(d.nv, kTabRows), nview), 256, 0, stream>>>(
+                siddon_bp_colpatch_kernel<<<dim3(patch_parts, nview), 256, 0, stream>>>(
                     wk, img + (b + k) * nimg, rowirr, pk, colw, roww, geo.det_center, geo.det_u, geo.det_v, geo.src, g,
                     d, wv);
                 CTP_LAUNCH_CHECK();
