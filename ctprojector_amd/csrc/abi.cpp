@@ -249,12 +249,12 @@ CTP_EXPORT int cupySiddonConeBackprojectionArbitrary(float* img, const float* pr
         cone_common(nBatches, nx, ny, nz, dx, dy, dz, cx, cy, cz, nu, nv, nview, du, dv, off_u, off_v, g, d);
         need_ptr(prj, "prj"); need_ptr(img, "img"); need_ptr(detCenter, "detCenter"); need_ptr(detU, "detU");
         need_ptr(detV, "detV"); need_ptr(src, "src");
+        touch();
         const size_t ng = 3 * nview;
-        std::vector<float> hc = host_copy(detCenter, ng), hu = host_copy(detU, ng), hv = host_copy(detV, ng),
-                           hs = host_copy(src, ng);
-        siddon_cone_bp(img, prj, ConeGeomDev{detCenter, detU, detV, src},
-                       ConeGeomHost{hc.data(), hu.data(), hv.data(), hs.data()}, (int)nBatches, g, d, (int)nview,
-                       cur_stream());
+        const ConeGeomDev geo{detCenter, detU, detV, src};
+        const std::vector<float> h = cone_geometry_to_host(geo, (int)nview, cur_stream());
+        siddon_cone_bp(img, prj, geo, ConeGeomHost{h.data(), h.data() + ng, h.data() + 2 * ng, h.data() + 3 * ng},
+                       (int)nBatches, g, d, (int)nview, cur_stream());
         sync();
     });
 }

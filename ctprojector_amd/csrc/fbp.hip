@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <cmath>
 #include <complex>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -720,20 +721,23 @@ void ramp_filter(float* out, const float* prj, int B, int nu, int nv, int nview,
         const RampFFTTables t = ramp_fft_tables(nu, da, filter, equispace, scale);
         Workspace& ws = workspace_for(stream);
         Plan pl;
-        pl.add<float>(t.N);
-        pl.add<float2>(t.N);
-        pl.add<float>(nu);
+        // spectrum, twiddles (the generic kernel's) and pre-weight in one upload
+        const bool three_pass = mode == 0 && t.N >= 1024;
+        const size_t ntw = three_pass ? 0 : 2 * (size_t)t.N;
+        std::vector<float> tab(t.N + ntw + nu);
+        std::memcpy(tab.data(), t.G.data(), sizeof(float) * t.N);
+        if (ntw > 0) std::memcpy(tab.data() + t.N, t.tw.data(), sizeof(float) * ntw);
+        std::memcpy(tab.data() + t.N + ntw, pw.data(), sizeof(float) * nu);
+        pl.add<float>(tab.size());
         ws.reserve(pl.bytes);
-        float* dG = ws.take_n<float>(t.N);
-        float2* dtw = ws.take_n<float2>(t.N);
-        float* dpw = ws.take_n<float>(nu);
-        CTP_CHECK(hipMemcpyAsync(dG, t.G.data(), sizeof(float) * t.N, hipMemcpyHostToDevice, stream));
-        CTP_CHECK(hipMemcpyAsync(dtw, t.tw.data(), sizeof(float2) * t.N, hipMemcpyHostToDevice, stream));
-        CTP_CHECK(hipMemcpyAsync(dpw, pw.data(), sizeof(float) * nu, hipMemcpyHostToDevice, stream));
+        float* dG = ws.take_n<float>(tab.size());
+        const float2* dtw = reinterpret_cast<const float2*>(dG + t.N);
+        const float* dpw = dG + t.N + ntw;
+        CTP_CHECK(hipMemcpyAsync(dG, tab.data(), sizeof(float) * tab.size(), hipMemcpyHostToDevice, stream));
         {
             TimedLaunch tl("ramp_filter", stream);
             const long pairs = ceil_div(nrows, 2);
-            if (mode == 0 && t.N >= 1024) {
+            if (three_pass) {
                 auto launch = [&](auto kernel, int block) {
                     const int rpb = block / (t.N / 16);
                     kernel<<<(unsigned)ceil_div(pairs, (long)rpb), block, 0, stream>>>(out, prj, dG, dpw, nrows, nu);
@@ -1236,16 +1240,21 @@ void fan_fbp_bp(float* img, const float* prj, const float* deg_host, int B, cons
     Workspace& ws = workspace_for(stream);
     Plan pl;
     pl.add<float>((size_t)nview * d.nu * cs);
-    pl.add<FBPView>(nview);
-    pl.add<SliceRow>(g.nz);
+    // view table and slice rows in one upload
+    static_assert(sizeof(FBPView) % 16 == 0 && sizeof(SliceRow) % 16 == 0, "tables follow each other");
+    const size_t vbytes = sizeof(FBPView) * nview;
+    std::vector<char> tab(vbytes + sizeof(SliceRow) * g.nz);
+    std::memcpy(tab.data(), views.data(), vbytes);
+    std::memcpy(tab.data() + vbytes, srow.data(), sizeof(SliceRow) * g.nz);
+    pl.add<char>(tab.size());
     if (groups > 1) pl.add<float>((size_t)groups * C * npix);
     ws.reserve(pl.bytes);
     float* q = ws.take_n<float>((size_t)nview * d.nu * cs);
-    FBPView* dviews = ws.take_n<FBPView>(nview);
-    SliceRow* dsrow = ws.take_n<SliceRow>(g.nz);
+    char* dtab = ws.take_n<char>(tab.size());
+    FBPView* dviews = reinterpret_cast<FBPView*>(dtab);
+    SliceRow* dsrow = reinterpret_cast<SliceRow*>(dtab + vbytes);
     float* part = groups > 1 ? ws.take_n<float>((size_t)groups * C * npix) : nullptr;
-    CTP_CHECK(hipMemcpyAsync(dviews, views.data(), sizeof(FBPView) * nview, hipMemcpyHostToDevice, stream));
-    CTP_CHECK(hipMemcpyAsync(dsrow, srow.data(), sizeof(SliceRow) * g.nz, hipMemcpyHostToDevice, stream));
+    CTP_CHECK(hipMemcpyAsync(dtab, tab.data(), tab.size(), hipMemcpyHostToDevice, stream));
     slices_to_channel_last(q, prj, dsrow, C, cs, g.nz, d, nview, stream);
     int lpc = tuning_get("fbp_bp_lanes_per_pixel", 4);
     if (lpc == 4 && CH % 16 != 0) lpc = 2;

@@ -1137,7 +1137,7 @@ __global__ __launch_bounds__(256) void siddon_bp_coltable_kernel(float* __restri
 // time: hardly any row is flagged, so a block's time is mostly that one load's
 // latency (a block per 8 rows, reading its flags one by one, took 70 us at
 // 256^3 / 720 views).  Where rows are flagged their rays cost far more than the
-// flags, so few views are split into more parts (128^3 and 60 views with flagged
+// flags, so few views are split into more parts (128^3, 180 views, with flagged
 // rows: 70 us, one exact ray's time; 190 us with one block per view).
 __global__ __launch_bounds__(256) void siddon_bp_colpatch_kernel(float* __restrict__ wtab, float* __restrict__ img,
                                                                  const int* __restrict__ rowirr,
@@ -2056,6 +2056,23 @@ void siddon_cone_fp(float* prj, const float* img, const ConeGeomDev& geo, int B,
             siddon_cone_fp_grid(prj + b * nprj, img + b * nimg + (size_t)z0 * per, geo, 1, cone_slab(g, z0, n), d,
                                 nview, stream);
         }
+}
+
+std::vector<float> cone_geometry_to_host(const ConeGeomDev& geo, int nview, hipStream_t stream) {
+    const int n = 3 * nview;
+    if (n <= 0) return {};
+    Workspace& ws = workspace_for(stream);
+    Plan pl;
+    pl.add<float>(4 * (size_t)n);
+    ws.reserve(pl.bytes);
+    float* all = ws.take_n<float>(4 * (size_t)n);
+    const float* part[4] = {geo.det_center, geo.det_u, geo.det_v, geo.src};
+    for (int k = 0; k < 4; k++)   // (copies, not a kernel: they refuse a null or too short array)
+        CTP_CHECK(hipMemcpyAsync(all + (size_t)k * n, part[k], sizeof(float) * n, hipMemcpyDeviceToDevice, stream));
+    std::vector<float> h(4 * (size_t)n);
+    CTP_CHECK(hipMemcpyAsync(h.data(), all, sizeof(float) * h.size(), hipMemcpyDeviceToHost, stream));
+    CTP_CHECK(hipStreamSynchronize(stream));
+    return h;
 }
 
 void siddon_cone_bp(float* img, const float* prj, const ConeGeomDev& geo, const ConeGeomHost& hgeo, int B,
