@@ -1917,14 +1917,18 @@ void dd2d_bp(float* img, const float* prj, const float* deg_host, int B, const G
 // non-finite detector value also reaches the pixels next to its footprint.
 // Bound by the L1's data path: a candidate is its record and its channels.  In
 // the fan beam half of the record is the source, read once per view and trace
-// instead (8 slices of 256^2, 492 views, 444 columns: 203 -> 146 us).
-struct FPTrace {           // one trace of a (view, column): edge lines r * (t - o) + b and the norm
-    float r1, r2, norm, pad;
-    float o1, b1, o2, b2;  // the source in the fan beam: the same for every column of a view
+// instead (8 slices of 256^2, 492 views, 444 columns: 203 -> 146 us; 144 with rows).
+//
+// Per view four rows of nu float4s, one per (trace, half): trace 0 along y (x
+// of row t), 1 along x (y of column t); half 0 {r1, r2, norm, -}, half 1 {o1,
+// b1, o2, b2}, the two edge lines r * (t - o) + b.  Rows, so that the columns
+// next to each other that a wavefront's pixels meet share cache lines.
+struct FPLine {            // a column's share of a view's rows
+    float4 v[4];
 };
-struct FPLine {            // per (view, column): trace along y (x of row t), trace along x (y of column t)
-    FPTrace tr[2];         // 32-byte aligned records: a candidate's trace is two 16-byte loads
-};
+__host__ __device__ inline size_t fp_line_row(int view, int tr, int half, int nu) {
+    return ((size_t)view * 4 + half * 2 + tr) * nu;
+}
 
 template <bool FAN>
 __global__ __launch_bounds__(256) void dd_fp_lines_kernel(FPLine* __restrict__ lines, const DDView* __restrict__ views,
@@ -1934,14 +1938,23 @@ __global__ __launch_bounds__(256) void dd_fp_lines_kernel(FPLine* __restrict__ l
     const DDView V = views[view];
     float2 s1, s2, d1, d2;
     const float a = fp_cell_edges<FAN>(iu, V, g, d, dsd, dso, s1, s2, d1, d2);
-    FPLine L{};
-    if (V.flags & 1)
-        L.tr[0] = FPTrace{(d1.x - s1.x) / (d1.y - s1.y), (d2.x - s2.x) / (d2.y - s2.y),
-                          V.wx * g.dy / fabsf(cosf(V.deg - a)), 0.f, s1.y, s1.x, s2.y, s2.x};
-    if (V.flags & 2)
-        L.tr[1] = FPTrace{(d1.y - s1.y) / (d1.x - s1.x), (d2.y - s2.y) / (d2.x - s2.x),
-                          (1.f - V.wx) * g.dx / fabsf(sinf(V.deg - a)), 0.f, s1.x, s1.y, s2.x, s2.y};
-    lines[(size_t)view * d.nu + iu] = L;
+    float4* rows = reinterpret_cast<float4*>(lines);
+    float4 l0 = make_float4(0.f, 0.f, 0.f, 0.f), l1 = l0;
+    if (V.flags & 1) {
+        l0 = make_float4((d1.x - s1.x) / (d1.y - s1.y), (d2.x - s2.x) / (d2.y - s2.y),
+                         V.wx * g.dy / fabsf(cosf(V.deg - a)), 0.f);
+        l1 = make_float4(s1.y, s1.x, s2.y, s2.x);
+    }
+    rows[fp_line_row(view, 0, 0, d.nu) + iu] = l0;
+    rows[fp_line_row(view, 0, 1, d.nu) + iu] = l1;
+    l0 = l1 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (V.flags & 2) {
+        l0 = make_float4((d1.y - s1.y) / (d1.x - s1.x), (d2.y - s2.y) / (d2.x - s2.x),
+                         (1.f - V.wx) * g.dx / fabsf(sinf(V.deg - a)), 0.f);
+        l1 = make_float4(s1.x, s1.y, s2.x, s2.y);
+    }
+    rows[fp_line_row(view, 1, 0, d.nu) + iu] = l0;
+    rows[fp_line_row(view, 1, 1, d.nu) + iu] = l1;
 }
 
 // G[view][u][c] = rev * sum over the detector rows of slice channel c of their
@@ -2005,7 +2018,6 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
     for (int j = 0; j < CH; j++) acc[j] = 0.f;
     for (int view = vbeg; view < vend; view++) {
         const DDView V = views[view];
-        const FPLine* __restrict__ Lv = lines + (size_t)view * d.nu;
         const float* __restrict__ Gv = G + (size_t)view * d.nu * cs + c0;
 #pragma unroll
         for (int tr = 0; tr < 2; tr++) {
@@ -2024,14 +2036,15 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
             const int n = tr == 0 ? g.nx : g.ny;
             const float lo = tr == 0 ? (float)ix : (float)iy;
             // (fan beam: the trace's origin is the source, one for all columns; half a record per candidate)
-            const float4 org = const_load(reinterpret_cast<const float4*>(&Lv[0].tr[tr]), 1);
+            const float4* __restrict__ L0 = reinterpret_cast<const float4*>(lines) + fp_line_row(view, tr, 0, d.nu);
+            const float4* __restrict__ L1 = reinterpret_cast<const float4*>(lines) + fp_line_row(view, tr, 1, d.nu);
+            const float4 org = const_load(L1, 0);
             for (int k = k0; k <= k1; k++) {
                 // the candidate's trace record and its channels load together
                 // (one memory round trip per candidate; taking candidates in
                 // pairs measured slower); a candidate whose weight is not
                 // positive adds 0 times its channels
-                const float4* __restrict__ lp = reinterpret_cast<const float4*>(&Lv[k].tr[tr]);
-                const float4 l0 = lp[0], l1 = FAN ? org : lp[1];   // r1 r2 norm - | o1 b1 o2 b2
+                const float4 l0 = L0[k], l1 = FAN ? org : L1[k];   // r1 r2 norm - | o1 b1 o2 b2
                 float q[CH];
                 const float* __restrict__ gp = Gv + (size_t)k * cs;
                 if constexpr (CH % 4 == 0) {
