@@ -1661,7 +1661,10 @@ template <int WU>
 static void launch_bp_planes(float* img, long istride, int nb, const WTabs& wtab, const float2* utab,
                              const float* qtab, const ConeViewBP* views, int nview, const Grid& g, const Det& d,
                              hipStream_t stream) {
-    const int nzr = tuning_get("cone_bp_zrun", nb == 1 ? 8 : 4);
+    // one run length for one and several volumes: a run's row coordinates start
+    // from its lowest plane, so another length rounds differently, and a volume
+    // has to come out the same alone and beside others of its geometry
+    const int nzr = tuning_get("cone_bp_zrun", 4);
     if (nb == 4 && nzr == 4) return launch_bp_planes_n<WU, 4, 4>(img, istride, wtab, utab, qtab, views, nview, g, d, stream);
     if (nb == 2 && nzr == 4) return launch_bp_planes_n<WU, 4, 2>(img, istride, wtab, utab, qtab, views, nview, g, d, stream);
     if (nb != 1) fail("cone backprojection: several volumes per launch need cone_bp_zrun 4");
