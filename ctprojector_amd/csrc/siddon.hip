@@ -1068,11 +1068,11 @@ __global__ __launch_bounds__(256) void siddon_bp_colaxes_kernel(float2* __restri
 // rules whatever the rounding: its weight is prj * |Q - S|, with hits decided
 // by the geometry of the chords themselves (a ray that misses the grid has no
 // chord in any voxel).  Rays near an axis direction take the FP64 path.
-// Fast-path weight of ray (view, iv, iu) (w = prj * |Q - S|), or -1 when the
-// ray is not regular and needs the FP64 path.
+// Fast-path weight of ray (view, iv, iu) (w = prj * |Q - S|, of any sign, or
+// not finite as prj is); 'regular' is false when the ray needs the FP64 path.
 __device__ inline float coltable_fast(long i, int iu, int iv, int view, const float* __restrict__ prj,
                                       const float2* __restrict__ colw, const float* __restrict__ roww,
-                                      const float* __restrict__ psrc, const Grid& g, const Det& d) {
+                                      const float* __restrict__ psrc, const Grid& g, const Det& d, bool& regular) {
     // Q - S (the axes kernel's FP64 values rounded to FP32: zero exactly when zero)
     const float2 cw = colw[(long)view * d.nu + iu];
     const float3 wf = make_float3(cw.x, cw.y, roww[(long)view * d.nv + iv]);
@@ -1086,9 +1086,9 @@ __device__ inline float coltable_fast(long i, int iu, int iv, int view, const fl
     const float rr = sqrtf(ex * ex + ey * ey + ez * ez);
     const float t0 = ((g.cx - Sf.x) * wf.x + (g.cy - Sf.y) * wf.y + (g.cz - Sf.z) * wf.z) * rL;
     const float frac = (L - fmaxf(t0 - rr, 0.f) - fmaxf(L - t0 - rr, 0.f)) * rL;
-    const bool regular = fabsf(wf.x) * frac > 1e-5f * g.dx && fabsf(wf.y) * frac > 1e-5f * g.dy &&
-                         fabsf(wf.z) * frac > 1e-5f * g.dz && frac > 0.f;
-    return regular ? prj[i] * L : -1.f;
+    regular = fabsf(wf.x) * frac > 1e-5f * g.dx && fabsf(wf.y) * frac > 1e-5f * g.dy &&
+              fabsf(wf.z) * frac > 1e-5f * g.dz && frac > 0.f;
+    return prj[i] * L;
 }
 
 // One thread per column and 8 consecutive rows of a view (grid: column
@@ -1112,10 +1112,14 @@ __global__ __launch_bounds__(256) void siddon_bp_coltable_kernel(float* __restri
     for (int r = 0; r < kTabRows + DUP - 1; r++) {
         float w = 0.f;
         if (r < nrow) {
-            w = coltable_fast(i0 + (long)r * d.nu, iu, iv0 + r, view, prj, colw, roww, psrc, g, d);
-            if (w < 0.f && r < kTabRows) rowirr[(long)view * d.nv + iv0 + r] = 1;
+            bool regular;
+            w = coltable_fast(i0 + (long)r * d.nu, iu, iv0 + r, view, prj, colw, roww, psrc, g, d, regular);
+            if (!regular) {
+                w = 0.f;
+                if (r < kTabRows) rowirr[(long)view * d.nv + iv0 + r] = 1;
+            }
         }
-        wr[r] = fmaxf(w, 0.f);
+        wr[r] = w;
     }
 #pragma unroll
     for (int r = 0; r < kTabRows; r++) {
@@ -1137,8 +1141,9 @@ __global__ __launch_bounds__(256) void siddon_bp_coltable_kernel(float* __restri
 // time: hardly any row is flagged, so a block's time is mostly that one load's
 // latency (a block per 8 rows, reading its flags one by one, took 70 us at
 // 256^3 / 720 views).  Where rows are flagged their rays cost far more than the
-// flags, so few views are split into more parts (128^3, 180 views, with flagged
-// rows: 70 us, one exact ray's time; 190 us with one block per view).
+// flags, so few views are split into more parts (128^3, 180 views, most rows
+// flagged: 70 us; 190 us with one block per view).  A row is flagged by its
+// geometry alone, never by the values measured on it.
 __global__ __launch_bounds__(256) void siddon_bp_colpatch_kernel(float* __restrict__ wtab, float* __restrict__ img,
                                                                  const int* __restrict__ rowirr,
                                                                  const float* __restrict__ prj,
@@ -1162,7 +1167,9 @@ __global__ __launch_bounds__(256) void siddon_bp_colpatch_kernel(float* __restri
             const int iv = list[r];
             for (int iu = threadIdx.x; iu < d.nu; iu += 256) {
                 const long i = ((long)view * d.nv + iv) * d.nu + iu;
-                if (coltable_fast(i, iu, iv, view, prj, colw, roww, psrc, g, d) >= 0.f) continue;
+                bool regular;
+                (void)coltable_fast(i, iu, iv, view, prj, colw, roww, psrc, g, d, regular);
+                if (regular) continue;
                 const float w = coltable_exact(i, iu, iv, view, true, img, prj, pdc, pdu, pdv, psrc, g, d);
                 for (int jv = 0; jv < dup && jv <= iv; jv++) wtab[(i - (long)jv * d.nu) * dup + jv] = w;
             }

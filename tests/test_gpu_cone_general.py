@@ -229,3 +229,44 @@ def test_bp_plane_form(oracle, tuning, case):
     e, d = rel_l2(a, oracle.siddon_cone_bp(g, y, *args)), rel_l2(a, b)
     _say(case, 'plane form against the oracle %.2e, against the windows %.2e' % (e, d))
     assert d < TOL and (e < TOL or case == 'axis_parallel')
+
+
+# Geometry of the tests below: no ray near an axis direction (so that no ray is
+# scattered atomically and results are compared bit for bit), several rows and
+# columns of the panel beside the volume, source heights on both sides of it.
+def _plane_case(nview=12, B=1, **over):
+    from ctprojector_amd.phantom import circular_cone_geometry
+    kw = dict(nx=23, ny=19, nz=37, dx=1.0, dy=1.0, dz=1.0, cx=0.4, cy=-0.3, cz=0.7, nu=44, nv=45, du=1.7, dv=1.7,
+              off_u=0.2, off_v=-0.4, dsd=300.0, dso=180.0)
+    kw.update(over)
+    g = Geo(**kw)
+    geo = circular_cone_geometry(nview, 180.0, 300.0, -6.0, 6.0, jitter=1.0, seed=5)
+    args = (geo.det_center, geo.det_u, geo.det_v, geo.src)
+    y = np.random.default_rng(8).uniform(-1, 1, size=[B, nview, g.nv, g.nu]).astype(np.float32)
+    return g, args, y
+
+
+@pytest.mark.parametrize('form', ['planes', 'windows', 'general'])
+def test_bp_signed_and_nan_rays(oracle, tuning, form):
+    """A ray is weighted alike whatever the sign of its value, so the
+    backprojection is odd bit for bit, and a NaN is not dropped: every voxel
+    that the ray crosses is NaN."""
+    from ctprojector_amd.projector.numpy import cone
+    from ctprojector_amd.projector.numpy.ct_projector import ct_projector
+    if form == 'windows':
+        tuning('cone_bp_planes', 2)
+    if form == 'general':
+        tuning('cone_bp_mode', 1)
+    g, args, y = _plane_case()
+    p = g.to(ct_projector())
+    a, b = cone.siddon_bp_arbitrary(p, y, *args), cone.siddon_bp_arbitrary(p, -y, *args)
+    e = rel_l2(a, oracle.siddon_cone_bp(g, y, *args))
+    _say(form, 'signed sinogram against the oracle %.2e' % e)
+    assert e < TOL and np.array_equal(a, -b)
+    unit = np.zeros_like(y)
+    unit[0, 3, 20, 25] = 1.0
+    met = oracle.siddon_cone_bp(g, unit, *args) > 1e-2   # chords of at least a hundredth of a voxel
+    y[0, 3, 20, 25] = np.nan
+    bad = np.isnan(cone.siddon_bp_arbitrary(p, y, *args))
+    _say(form, 'voxels met by the NaN ray', int(met.sum()), 'NaN voxels', int(bad.sum()))
+    assert met.sum() > 10 and bad[met].all()
