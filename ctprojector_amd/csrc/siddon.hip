@@ -1553,6 +1553,48 @@ __device__ __forceinline__ void bp_view_planes(float* acc, const ConeViewBP& cv,
     }
 }
 
+// One voxel of the plane form, ray by ray, with rays that have no chord in it
+// left out: the sums of bp_planes_run take weights times differences of chords
+// (a ray's part above a plane less its part above the next), which for an
+// infinite weight is NaN, also in voxels that the ray does not meet.  Voxels
+// that come out NaN are summed again here, so that weights that are not finite
+// reach the voxels their rays cross and no others.
+template <int WU>
+__device__ float bp_planes_voxel(const float* __restrict__ wtab, const float2* __restrict__ utab,
+                                 const float* __restrict__ qtab, const ConeViewBP* __restrict__ views, int nview,
+                                 int nu, int nv, int ix, int iy, int iz) {
+    const size_t nuv = (size_t)nu * nv;
+    float sum = 0.f;
+    for (int view = 0; view < nview; view++) {
+        const ConeViewBP cv = const_load(views, view);
+        PlaneColumn<WU> P;
+        bp_planes_column<WU>(P, cv, utab + (size_t)view * nu, nu, ix, iy, ix + 0.5f, iy + 0.5f);
+        const float g1 = P.v[2 * WU], g0 = P.v[2 * WU + 1];
+        const int u0 = __float_as_int(P.v[2 * WU + 2]) / 4;
+        float p[2];                                    // the voxel's planes: heights, first rows not wholly below
+        int first[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            p[k] = (float)(iz + k) - cv.sz;
+            const float v = fminf(fmaf(p[k], g1, cv.v0), fmaf(p[k], g0, cv.v0)) + kRowBias;
+            first[k] = (int)(v - kRowBias);
+        }
+        for (int r = max(first[0], 0); r <= min(first[1], nv - 1); r++) {
+            const size_t row = (size_t)view * nv + (cv.flip ? nv - 1 - r : r);
+            const float q = qtab[row];
+            const float* __restrict__ w = wtab + view * nuv + (row - (size_t)view * nv) * nu + u0;
+#pragma unroll
+            for (int j = 0; j < WU; j++) {
+                const float lo = P.v[2 * j], hi = P.v[2 * j + 1];
+                auto above = [&](float h) { return fabsf((q > 0.f ? hi : lo) - __builtin_amdgcn_fmed3f(h * q, lo, hi)); };
+                const float chord = (r == first[0] ? above(p[0]) : hi - lo) - (r == first[1] ? above(p[1]) : 0.f);
+                if (chord > 0.f) sum = fmaf(w[j], chord, sum);
+            }
+        }
+    }
+    return sum;
+}
+
 // weight tables (per-call window layout) of up to 4 volumes of one geometry
 struct WTabs {
     const float* p[4];
@@ -1634,12 +1676,26 @@ __device__ __forceinline__ void bp_planes_block(PlaneShare<WU>& sh, float* __res
         }
     }
     if (ix >= g.nx || iy >= g.ny) return;
+    unsigned bad = 0;   // NaN sums, by k * NB + b
 #pragma unroll
     for (int k = 0; k < NZR; k++) {
         const int iz = iz0 + k;
         if (iz < g.nz)
 #pragma unroll
-            for (int b = 0; b < NB; b++) img[b * istride + ((size_t)iz * g.ny + iy) * g.nx + ix] += acc[k * NB + b];
+            for (int b = 0; b < NB; b++) {
+                const float a = acc[k * NB + b];
+                if (__builtin_isnan(a)) bad |= 1u << (k * NB + b);
+                else img[b * istride + ((size_t)iz * g.ny + iy) * g.nx + ix] += a;
+            }
+    }
+    while (bad != 0) {
+        const int i = __builtin_ctz(bad), iz = iz0 + i / NB, b = i % NB;
+        bad &= bad - 1;
+        const float* wt = wtab.p[0];
+#pragma unroll
+        for (int c = 1; c < NB; c++) wt = b == c ? wtab.p[c] : wt;
+        img[b * istride + ((size_t)iz * g.ny + iy) * g.nx + ix] +=
+            bp_planes_voxel<WU>(wt, utab, qtab, views, nview, nu, nv, ix, iy, iz);
     }
 }
 
