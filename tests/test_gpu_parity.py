@@ -619,3 +619,68 @@ def test_tomo_window_form(oracle, case):
     bad = np.isnan(tomo.distance_driven_fp(p, lit, dc, src))
     # (the lit voxel lies beside the truncated panel: no ray meets it)
     assert met.any() == (case != 'truncated') and bad[met].all() and bad.sum() <= met.sum() + 2
+
+
+@pytest.mark.parametrize('nz', [1, 2, 3, 4])
+@pytest.mark.parametrize('case', ['fan', 'fan_fbp', 'fan_wide', 'parallel', 'parallel_fbp', 'parallel_wide'])
+def test_dd_window_bp_not_finite(oracle, case, nz):
+    """A detector cell that is not finite reaches the pixels whose footprints
+    meet it, and no others, in the window form of the DD backprojectors (up to
+    4 slices; 'wide' footprints of more than 2 cells are walked).  Pixels met
+    by less than a thousandth of a cell may come out either way."""
+    beam = case.split('_')[0]
+    kw = dict(nx=61, ny=45, nz=nz, dx=1.0, dy=1.0, dz=1.0, cx=1.3, cy=-0.6, nu=97, nv=nz, du=1.17, dv=1.0, off_u=0.31)
+    if beam == 'fan':
+        kw.update(dsd=400.0, dso=240.0, du=1.9)
+    if case.endswith('wide'):
+        kw.update(du=0.35 * kw['du'], nu=260)
+    g = Geo(**kw)
+    ang = (np.arange(19) * (2 if beam == 'fan' else 1) * np.pi / 19 + 0.013).astype(np.float32)
+    m = fan if beam == 'fan' else parallel
+    ref = oracle.dd_fan_bp if beam == 'fan' else oracle.dd_par_bp
+    is_fbp = case.endswith('fbp')
+    y = np.random.default_rng(3).uniform(-1, 1, size=[1, 19, nz, g.nu]).astype(np.float32)
+    unit = np.zeros_like(y)
+    unit[0, 5, nz - 1, g.nu // 2 + 3] = unit[0, 11, 0, g.nu // 2 - 6] = 1.0
+    w = np.abs(ref(g, unit, ang, is_fbp=is_fbp))
+    p = _proj(g)
+    for value in (np.nan, np.inf):
+        bad = ~np.isfinite(m.distance_driven_bp(p, np.where(unit > 0, np.float32(value), y), ang, is_fbp=is_fbp))
+        print('dd window bp', case, nz, value, int((w > 0).sum()), int(bad.sum()))
+        assert (w > 0).sum() > 20 and bad[w > 1e-3 * w.max()].all() and not bad[(w == 0) & ~_beside(w > 0)].any()
+        assert bad.sum() <= (w > 0).sum() + 4
+
+
+def _beside(a):
+    """Cells of the last two axes next to a true one."""
+    b = np.zeros_like(a)
+    b[..., 1:, :] |= a[..., :-1, :]
+    b[..., :-1, :] |= a[..., 1:, :]
+    b[..., 1:] |= a[..., :-1]
+    b[..., :-1] |= a[..., 1:]
+    return b
+
+
+@pytest.mark.parametrize('case', ['coarse', 'fine', 'wide', 'truncated'])
+def test_tomo_window_bp_not_finite(oracle, case):
+    """A detector cell that is not finite reaches the voxels whose boxes meet it,
+    and no others, in the window form of the tomosynthesis backprojector."""
+    kw = dict(nx=37, ny=29, nz=11, dx=1.0, dy=1.0, dz=1.0, cz=20.0, nu=43, nv=39, du=1.03, dv=0.97, off_u=0.2)
+    if case == 'fine':
+        kw.update(du=0.7, dv=0.6, nu=61, nv=57)
+    if case == 'wide':
+        kw.update(du=0.3, dv=0.4, nu=141, nv=99)
+    if case == 'truncated':
+        kw.update(nu=20, nv=11, cx=6.0)
+    g = Geo(**kw)
+    t = np.linspace(-0.4, 0.4, 5)
+    src = np.stack([300 * np.sin(t), 5 * np.ones_like(t), 300 * np.cos(t) + 20], 1).astype(np.float32)
+    dc = np.stack([0 * t, 0 * t, 0 * t - 10], 1).astype(np.float32)
+    y = np.random.default_rng(9).uniform(-1, 1, size=[1, 5, g.nv, g.nu]).astype(np.float32)
+    unit = np.zeros_like(y)
+    unit[0, 2, g.nv // 2, g.nu // 2] = unit[0, 3, 0, g.nu - 1] = 1.0   # inside, and the panel's corner
+    w = np.abs(oracle.dd_tomo_bp(g, unit, dc, src))
+    for value in (np.nan, np.inf):
+        bad = ~np.isfinite(tomo.distance_driven_bp(_proj(g), np.where(unit > 0, np.float32(value), y), dc, src))
+        print('tomo window bp', case, value, int((w > 0).sum()), int(bad.sum()))
+        assert (w > 0).sum() > 5 and bad[w > 1e-3 * w.max()].all() and bad.sum() <= (w > 0).sum() + 4
