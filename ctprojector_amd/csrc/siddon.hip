@@ -719,14 +719,15 @@ static ConeBPPlan make_cone_bp_plan(const ConeGeomHost& h, const Grid& g, const 
         double tmax = 0;
         for (int cc = 0; cc < 4; cc++)
             tmax = std::max(tmax, (Pw[3] + ((cc & 1) ? g.nx * Pw[0] : 0.0) + ((cc & 2) ? g.ny * Pw[1] : 0.0)) * scale);
-        // the kernel's row coordinates are off by a few 1e-7 of the largest
-        const double slack = std::max(1e-3, 2e-6 * (d.nv + std::fabs(v0)));
-        const double vfar = std::max(std::fabs(v0 + 1), std::fabs(d.nv - v0));
-        if (!(kv != 0) || !(vfar * 2 * ht / tmin + 3 * slack < 1)) plan.planes = false;
         // rows of any plane stay within 22 bits and their byte offsets within 31
         const double pfar = std::max(std::fabs(S[2] - x0[2]), std::fabs(x0[2] + g.nz * dd[2] - S[2])) / dd[2] + 16;
         const double rfar = std::fabs(v0) + d.nv + std::fabs(kv) * pfar / tmin + 2;
         if (!(rfar < 2e6 && rfar * d.nu < 5e8)) plan.planes = false;
+        // the kernel's row coordinates are off by a few 1e-7 of the detector's
+        // and of the lowest plane's, on which they are all built
+        const double slack = std::max(1e-3, std::max(2e-6 * (d.nv + std::fabs(v0)), 3e-7 * rfar));
+        const double vfar = std::max(std::fabs(v0 + 1), std::fabs(d.nv - v0));
+        if (!(kv != 0) || !(vfar * 2 * ht / tmin + 3 * slack < 1)) plan.planes = false;
         // rows met by a block's 8 x 8 columns (of which the last may reach 8
         // past the grid) and kPlaneSpan planes, and 5 spare (the base's 2,
         // roundings and ends): they fit the stretch staged in LDS
@@ -1393,34 +1394,40 @@ typedef __attribute__((address_space(3))) float lds_float;
 
 // What a view gives every plane of a run.
 struct PlaneRun {
-    float g, c;            // row coordinate of plane k: c + k g (MIXED: at one end of the span, c1 + k g1 at the other)
-    float g1, c1;
+    float sz;              // source height, voxels
+    float g, c;            // row coordinate of the plane at height z: c + z g at the end of the span where it is lowest
+    float g1, c1;          // (MIXED: for the planes on the other side of the source: c1 + z g1)
+    bool above;            // the run's first plane is not below the source
     int wb;                // byte offset of the weight of row -2^22 in the lane's first column
     int stride;            // bytes per row
     unsigned qb;           // LDS address of the staged row table's (biased) row 0
 
-    // first row not wholly below plane k, biased
+    // first row not wholly below the plane at height z, biased
     template <bool MIXED>
-    __device__ __forceinline__ float row(int k) const {
-        float v = k == 0 ? c : fmaf((float)k, g, c);
-        if (MIXED) v = fminf(v, k == 0 ? c1 : fmaf((float)k, g1, c1));
-        return v + kRowBias;
+    __device__ __forceinline__ float row(float z) const {
+        const bool other = MIXED && (z >= sz) != above;
+        return fmaf(z, other ? g1 : g, other ? c1 : c) + kRowBias;
     }
 };
 
 template <int WU>
 struct PlaneColumn;
 
+// z: height of each plane in voxels (uniform).  A plane's row and crossings are
+// computed from that height alone, by the same operations in every form (the
+// contraction is off for the same reason): a voxel comes out the same bit for
+// bit whichever run, launch or number of volumes it is computed in.
 template <int WU, int NZR, int NB, bool MIXED>
 __device__ __forceinline__ void bp_planes_run(float* acc, const __amdgpu_buffer_rsrc_t* rw, const PlaneColumn<WU>& P,
-                                              const PlaneRun& R, float p0, bool above) {
+                                              const PlaneRun& R, const float* z) {
+#pragma clang fp contract(off)
     float q[NZR + 1], w[NZR + 1][NB][WU], last = 0.f;
     bool fresh[NZR + 1];                               // r_k != r_{k-1} (kept as lane masks)
 #pragma unroll
     for (int k = 0; k <= NZR; k++) {
         // rows below 0 and above nv - 1 weigh nothing: their loads are out of
         // the buffers' range and return 0
-        const float rf = R.template row<MIXED>(k);
+        const float rf = R.template row<MIXED>(z[k]);
         const int r = __float_as_int(rf);
         fresh[k] = k > 0 && rf != last;
         last = rf;
@@ -1433,23 +1440,26 @@ __device__ __forceinline__ void bp_planes_run(float* acc, const __amdgpu_buffer_
     float end[WU], len[WU];
 #pragma unroll
     for (int j = 0; j < WU; j++) {
-        end[j] = above ? P.v[2 * j + 1] : P.v[2 * j];
+        end[j] = R.above ? P.v[2 * j + 1] : P.v[2 * j];
         len[j] = P.v[2 * j + 1] - P.v[2 * j];
     }
 #pragma unroll
     for (int k = 0; k <= NZR; k++) {
-        const float p = p0 + (float)k;                 // plane height above the source, voxels
-        const float t = p * q[k];
+        const float t = (z[k] - R.sz) * q[k];          // plane height above the source times 1/w_z
         float a[WU];
 #pragma unroll
         for (int j = 0; j < WU; j++) {
             const float lo = P.v[2 * j], hi = P.v[2 * j + 1];
-            if (MIXED) a[j] = __builtin_amdgcn_fmed3f(fmaf(-p, fabsf(q[k]), q[k] > 0.f ? hi : -lo), 0.f, len[j]);
-            else a[j] = fabsf(end[j] - __builtin_amdgcn_fmed3f(t, lo, hi));
+            a[j] = fabsf((MIXED ? (q[k] > 0.f ? hi : lo) : end[j]) - __builtin_amdgcn_fmed3f(t, lo, hi));
         }
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             float s = w[k][b][0] * a[0], f = w[k][b][0] * len[0];
+            if constexpr (WU == 1) {
+                if (k < NZR) acc[k * NB + b] = fmaf(w[k][b][0], a[0], acc[k * NB + b]);
+                if (k > 0) acc[(k - 1) * NB + b] += fmaf(-w[k][b][0], a[0], fresh[k] ? f : 0.f);
+                continue;
+            }
 #pragma unroll
             for (int j = 1; j < WU; j++) {
                 s = fmaf(w[k][b][j], a[j], s);
@@ -1464,11 +1474,11 @@ __device__ __forceinline__ void bp_planes_run(float* acc, const __amdgpu_buffer_
 // Rows wholly inside a voxel besides r_{k+1} (where a voxel may hold more than one).
 template <int WU, int NZR, int NB, bool MIXED>
 __device__ __forceinline__ void bp_planes_more(float* acc, const __amdgpu_buffer_rsrc_t* rw, const PlaneColumn<WU>& P,
-                                               const PlaneRun& R, int extra) {
-    int last = __float_as_int(R.template row<MIXED>(0));
+                                               const PlaneRun& R, const float* z, int extra) {
+    int last = __float_as_int(R.template row<MIXED>(z[0]));
 #pragma unroll
     for (int k = 1; k <= NZR; k++) {
-        const int r = __float_as_int(R.template row<MIXED>(k));
+        const int r = __float_as_int(R.template row<MIXED>(z[k]));
         const int more = r - last - 1;
         last = r;
         if (__any(more > 0))
@@ -1520,22 +1530,22 @@ __device__ __forceinline__ void bp_planes_column(PlaneColumn<WU>& P, const ConeV
 template <int WU, int NZR, int NB>
 __device__ __forceinline__ void bp_view_planes(float* acc, const ConeViewBP& cv, const PlaneColumn<WU>& P,
                                                const float* const* wt, const float* __restrict__ qrow, int rbase,
-                                               int nu, int nv, int iz0) {
+                                               int nu, int nv, const float* z) {
     __amdgpu_buffer_rsrc_t rw[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++)
         rw[b] = __builtin_amdgcn_make_buffer_rsrc((void*)wt[b], (short)0, 4 * nu * nv, 0x00020000);
-    const float p0 = (float)iz0 - cv.sz;
-    const bool above = p0 >= 0.f;                                             // (uniform)
+    const bool above = z[0] >= cv.sz;                                         // (uniform)
     // the candidate rays of planes near the source's height may rise or fall
-    const bool mixed = p0 < cv.pm && p0 + (float)NZR > -cv.pm;
+    const bool mixed = z[0] - cv.sz < cv.pm && z[NZR] - cv.sz > -cv.pm;
     const float g1 = P.v[2 * WU], g0 = P.v[2 * WU + 1];
     PlaneRun R;
-    // the row coordinate at the end of the span where it is lowest
+    R.sz = cv.sz;
+    R.above = above;
     R.g = above ? g1 : g0;
-    R.c = fmaf(p0, R.g, cv.v0);
     R.g1 = above ? g0 : g1;
-    R.c1 = fmaf(p0, R.g1, cv.v0);
+    R.c = fmaf(-cv.sz, R.g, cv.v0);
+    R.c1 = fmaf(-cv.sz, R.g1, cv.v0);
     R.stride = cv.flip ? -4 * nu : 4 * nu;
     const unsigned bias = 1u << 22;
     R.wb = (int)((unsigned)__float_as_int(P.v[2 * WU + 2]) +
@@ -1545,11 +1555,11 @@ __device__ __forceinline__ void bp_view_planes(float* acc, const ConeViewBP& cv,
     // rounding of the row coordinates): no voxel holds a row besides r_{k+1}
     const bool more = cv.extra > 0 && __any(g0 > 0.999f);
     if (!mixed) {
-        bp_planes_run<WU, NZR, NB, false>(acc, rw, P, R, p0, above);
-        if (more) bp_planes_more<WU, NZR, NB, false>(acc, rw, P, R, cv.extra);
+        bp_planes_run<WU, NZR, NB, false>(acc, rw, P, R, z);
+        if (more) bp_planes_more<WU, NZR, NB, false>(acc, rw, P, R, z, cv.extra);
     } else {
-        bp_planes_run<WU, NZR, NB, true>(acc, rw, P, R, p0, above);
-        if (more) bp_planes_more<WU, NZR, NB, true>(acc, rw, P, R, cv.extra);
+        bp_planes_run<WU, NZR, NB, true>(acc, rw, P, R, z);
+        if (more) bp_planes_more<WU, NZR, NB, true>(acc, rw, P, R, z, cv.extra);
     }
 }
 
@@ -1576,8 +1586,8 @@ __device__ float bp_planes_voxel(const float* __restrict__ wtab, const float2* _
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             p[k] = (float)(iz + k) - cv.sz;
-            const float v = fminf(fmaf(p[k], g1, cv.v0), fmaf(p[k], g0, cv.v0)) + kRowBias;
-            first[k] = (int)(v - kRowBias);
+            const float z = (float)(iz + k), g = z >= cv.sz ? g1 : g0;
+            first[k] = (int)((fmaf(z, g, fmaf(-cv.sz, g, cv.v0)) + kRowBias) - kRowBias);
         }
         for (int r = max(first[0], 0); r <= min(first[1], nv - 1); r++) {
             const size_t row = (size_t)view * nv + (cv.flip ? nv - 1 - r : r);
@@ -1599,6 +1609,19 @@ __device__ float bp_planes_voxel(const float* __restrict__ wtab, const float2* _
 struct WTabs {
     const float* p[4];
 };
+
+// A wave-uniform float in a scalar register.  (The compiler turns the builtin
+// of a uniform conversion back into a vector register; the wait states are the
+// instruction's own, which it does not add around inline code.)
+__device__ inline float scalar_register(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r;
+    asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1\n\ts_nop 3" : "=s"(r) : "v"(x));
+    return r;
+#else
+    return x;
+#endif
+}
 
 // One block of the plane form: 8 x 8 voxel columns x 4 runs of NZR slices, one
 // run per wavefront, img += A^T y over all views, for NB volumes (volume b at
@@ -1625,9 +1648,11 @@ __device__ __forceinline__ void bp_planes_block(PlaneShare<WU>& sh, float* __res
     const int iy = by * 8 + (lane >> 3);
     const int iz0 = (bz * 4 + wave) * NZR;
     const float xc = ix + 0.5f, yc = iy + 0.5f;
-    float acc[NZR * NB];
+    float acc[NZR * NB], z[NZR + 1];
 #pragma unroll
     for (int k = 0; k < NZR * NB; k++) acc[k] = 0.f;
+#pragma unroll
+    for (int k = 0; k <= NZR; k++) z[k] = scalar_register((float)(iz0 + k));   // over all views
     const size_t nuv = (size_t)nu * nv;
     int buf = 0;
     for (int v0 = 0; v0 < nview; v0 += 4, buf ^= 1) {
@@ -1672,7 +1697,7 @@ __device__ __forceinline__ void bp_planes_block(PlaneShare<WU>& sh, float* __res
 #pragma unroll
             for (int b = 0; b < NB; b++) wt[b] = wtab.p[b] + view * nuv;
             bp_view_planes<WU, NZR, NB>(acc, cv, P, wt, sh.q[buf][t], __builtin_amdgcn_readfirstlane(sh.rbase[buf][t]),
-                                        nu, nv, iz0);
+                                        nu, nv, z);
         }
     }
     if (ix >= g.nx || iy >= g.ny) return;

@@ -308,3 +308,46 @@ def test_bp_planes_not_finite(oracle, tuning, value):
     b.prj[0].copy_(torch.from_numpy(y[1]))
     b.backward()
     check('plan', b.img[0].cpu().numpy(), ref[1], met[1])
+
+
+@pytest.mark.parametrize('case', ['default', 'narrow', 'three_columns', 'fine_columns', 'more_rows', 'flipped', 'tall'])
+def test_bp_planes_bits_do_not_depend_on_the_run(tuning, case):
+    """The plane form gives a voxel the same bits in z-runs of 1, 2, 4 and 8
+    slices, alone and among 2, 4 or 5 volumes of one geometry, and the batch
+    plan in z-runs of 2, 4 and 8 (which its autotuner chooses by time), with
+    planes on both sides of the source and candidate windows of 1 to 4 columns;
+    and it is the plane form that runs: the windows round otherwise."""
+    import torch
+    from types import SimpleNamespace
+    from ctprojector_amd.batched import ConeBatch, ConeJob
+    from ctprojector_amd.projector.numpy import cone
+    from ctprojector_amd.projector.numpy.ct_projector import ct_projector
+    over = {'default': {}, 'narrow': dict(du=3.4, nu=22), 'three_columns': dict(du=1.0, nu=75),
+            'fine_columns': dict(du=0.75, nu=100), 'flipped': {},
+            'more_rows': dict(dz=1.5, nz=21, dv=1.1, nv=70), 'tall': dict(nz=301, cz=60.0, nv=30)}[case]
+    g, args, y = _plane_case(B=5, **over)
+    if case == 'flipped':
+        args = (args[0], args[1], -args[2], args[3])
+    p = g.to(ct_projector())
+    ref = cone.siddon_bp_arbitrary(p, y[:1], *args)
+    for b in (2, 4, 5):
+        out = cone.siddon_bp_arbitrary(p, np.concatenate([y[1:b], y[:1]]), *args)
+        assert np.array_equal(out[-1:], ref), '%d volumes' % b
+        out = cone.siddon_bp_arbitrary(p, y[:b], *args)
+        assert np.array_equal(out[:1], ref), '%d volumes' % b
+    geo = SimpleNamespace(det_center=args[0], det_u=args[1], det_v=args[2], src=args[3])
+    plans = []
+    for z in (1, 2, 4, 8):
+        tuning('cone_bp_zrun', z)
+        assert np.array_equal(cone.siddon_bp_arbitrary(p, y[:1], *args), ref), 'z-run %d' % z
+        if z > 1:
+            b = ConeBatch([ConeJob(p, geo)])
+            b.prj[0].copy_(torch.from_numpy(y[0]))
+            b.backward()
+            plans.append(b.img[0].clone())
+    assert torch.equal(plans[0], plans[1]) and torch.equal(plans[0], plans[2])
+    tuning('cone_bp_zrun', 0)
+    tuning('cone_bp_planes', 2)
+    windows = cone.siddon_bp_arbitrary(p, y[:1], *args)
+    _say(case, 'voxels that the windows round otherwise: %.2f' % (windows != ref).mean())
+    assert (windows != ref).any() and rel_l2(windows, ref) < TOL
