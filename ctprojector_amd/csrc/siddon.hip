@@ -1749,13 +1749,19 @@ template <int WU>
 static void launch_bp_planes(float* img, long istride, int nb, const WTabs& wtab, const float2* utab,
                              const float* qtab, const ConeViewBP* views, int nview, const Grid& g, const Det& d,
                              hipStream_t stream) {
-    // one run length for one and several volumes: a run's row coordinates start
-    // from its lowest plane, so another length rounds differently, and a volume
-    // has to come out the same alone and beside others of its geometry
-    const int nzr = tuning_get("cone_bp_zrun", 4);
+    // Runs of 8 slices for one volume share a run's ends among more voxels
+    // (256^3 / 720 views: 9.3 against 10.1 ms; 128^3 / 180: kernel 318 against
+    // 409 us), where blocks of four such runs are mostly full and number at
+    // least four a CU (256^2 x 48 / 360 views 1.09 against 1.04 ms, 96^3 / 180
+    // 365 against 332 us: runs of 4); runs of 2 where four of them hold the
+    // volume (512^2 x 6 / 180: 460 against 483 us).  A voxel's bits are the same
+    // in all.
+    const long span = 32L * ceil_div(g.nz, 32);   // slices of the blocks of runs of 8
+    const bool full = 4L * g.nz > 3 * span && (long)ceil_div(g.nx, 8) * ceil_div(g.ny, 8) * (span / 32) >= 4 * 256;
+    const int nzr = tuning_get("cone_bp_zrun", nb > 1 ? 4 : full ? 8 : g.nz <= 8 ? 2 : 4);
     if (nb == 4 && nzr == 4) return launch_bp_planes_n<WU, 4, 4>(img, istride, wtab, utab, qtab, views, nview, g, d, stream);
     if (nb == 2 && nzr == 4) return launch_bp_planes_n<WU, 4, 2>(img, istride, wtab, utab, qtab, views, nview, g, d, stream);
-    if (nb != 1) fail("cone backprojection: several volumes per launch need cone_bp_zrun 4");
+    if (nb != 1) fail("cone backprojection: several volumes per launch need cone_bp_zrun 4");   // (the caller's rule)
     switch (nzr) {
         case 1: launch_bp_planes_n<WU, 1, 1>(img, istride, wtab, utab, qtab, views, nview, g, d, stream); break;
         case 2: launch_bp_planes_n<WU, 2, 1>(img, istride, wtab, utab, qtab, views, nview, g, d, stream); break;
@@ -2780,7 +2786,21 @@ ConePlan::ConePlan(const std::vector<ConeJobSpec>& specs, bool autotune) : impl_
     if (mode != 0 && mode != 1) fail("cone_fp_mode must be 0 or 1");
     P.tu = mode == 0 ? 0 : tuning_get("cone_fp_tile_u", 32);
     P.order = fp_xcd_order(mode);
-    P.nzr = tuning_get("cone_bp_zrun", 4);
+    // plane form's z-run, as launch_bp_planes chooses it, over all jobs (twelve
+    // jobs of 48^3 to 96^3: plan 1.26 ms with runs of 8, 1.28 with 4; four jobs of
+    // 40^3 to 96^3, 682 blocks of runs of 8: 236 us against 190; four jobs of
+    // 128^2 x 2: 207 us with runs of 2, 225 with 4)
+    long slices = 0, held = 0, tallest = 0;
+    for (const ConeJobDev& J : P.jobs)
+        if (J.wv == 0) {
+            const long tiles = (long)ceil_div(J.g.nx, 8) * ceil_div(J.g.ny, 8);
+            slices += tiles * J.g.nz;
+            held += tiles * 32 * ceil_div(J.g.nz, 32);
+            tallest = std::max(tallest, (long)J.g.nz);
+        }
+    P.nzr = tuning_get("cone_bp_zrun", 4 * slices > 3 * held && held / 32 >= 4 * 256 ? 8
+                                       : tallest > 0 && tallest <= 8                 ? 2
+                                                                                     : 4);
     if (P.tu != 0 && P.tu != 8 && P.tu != 16 && P.tu != 32 && P.tu != 64)
         fail("cone_fp_tile_u must be 8, 16, 32 or 64");
     if (P.nzr != 2 && P.nzr != 4 && P.nzr != 8) fail("cone plan: cone_bp_zrun must be 2, 4 or 8");
