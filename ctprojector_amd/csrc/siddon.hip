@@ -594,6 +594,8 @@ struct ConeBPPlan {
     int wu = 0, wv = 0;
     int near_view = -1;     // a view whose source is inside or too close to the volume (no bounded window)
     bool planes = true;     // column mode: every view allows the plane form
+    double rows = 0;        // most detector rows per voxel height
+    double spread = 0;      // most rows by which a plane's row differs among a block's columns
 };
 
 // Builds the per-view projective maps in FP64 from host geometry.  A view whose
@@ -732,8 +734,10 @@ static ConeBPPlan make_cone_bp_plan(const ConeGeomHost& h, const Grid& g, const 
         // past the grid) and kPlaneSpan planes, and 5 spare (the base's 2,
         // roundings and ends): they fit the stretch staged in LDS
         const double edge = tmin - 16 * ht;
-        if (!(edge > 0) || !(kPlaneSpan * ka / edge + ka * pfar / edge * (16 * ht / edge) + 5 < kPlaneRows))
-            plan.planes = false;
+        const double spread = ka * pfar / edge * (16 * ht / edge);
+        if (!(edge > 0) || !(kPlaneSpan * ka / edge + spread + 5 < kPlaneRows)) plan.planes = false;
+        plan.rows = std::max(plan.rows, ka / tmin);
+        plan.spread = std::max(plan.spread, spread);
         cv.flip = kv < 0 ? 1 : 0;
         cv.v0 = (float)((kv < 0 ? d.nv - 1 - v0 : v0) - slack + 0.5);
         cv.kv = (float)ka;
@@ -1869,6 +1873,28 @@ static bool plane_form(const ConeBPPlan& plan, const Det& d) {
            tuning_get("cone_bp_planes", 1) != 2;
 }
 
+// A single call keeps the windows where they are faster (a batch plan does not:
+// its jobs fill the chip together, and jobs of two forms are two launches):
+// - up to 4 slices whose columns fill the chip with the windows' blocks of
+//   16 x 16 (three blocks a CU): most wavefronts of a plane block have no
+//   slice to work on (448^2 x 4 / 180 views: windows 302 us, planes 368; 512^2
+//   302 against 447; but 384^2 x 4, 576 blocks, 418 against 363);
+// - voxels that often hold whole rows besides the crossing ones, which the
+//   plane form adds one by one.  Windows of two rows: more than 1.25 rows per
+//   voxel height, and rows that differ so much among a block's columns that some
+//   column nearly always has one (1.38 rows, spread 3.0, 200^3 / 90 views:
+//   windows 901 us, planes 974; 1.33 rows, spread 2.1, 160^2 x 128: 526 against
+//   461; 1.28 rows, spread 2.6, 200^3: 896 against 919).  Windows of four rows:
+//   three such rows (200^2 x 128 / 180 views 2.18 against 2.36 ms; with two,
+//   2.26 against 1.87).
+// The rule reads the geometry alone, never how many volumes share a launch:
+// a volume comes out the same alone and beside others.
+static bool planes_pay(const ConeBPPlan& plan, const Grid& g) {
+    const bool thin = g.nz <= 4 && (long)ceil_div(g.nx, 16) * ceil_div(g.ny, 16) >= 3 * 256;
+    const bool dense = (plan.wv <= 2 && plan.rows > 1.25 && plan.spread > 2.4) || plan.rows > 3;
+    return !thin && !dense;
+}
+
 template <int WU, int WV, int NZR>
 static void launch_bp_n(float* img, const float4* table, const ConeViewBP* views, int nview, const Grid& g,
                         const Det& d, hipStream_t stream) {
@@ -1982,7 +2008,7 @@ static void siddon_cone_bp_grid(float* img, const float* prj, const ConeGeomDev&
     wv = std::min(std::max(wv, 1), d.nv);
     const bool col = bp_mode == 0 && column_mode(hgeo, plan, nview) && d.nu < (1 << 20);
     // plane form: one weight per ray (table height 1)
-    const bool planes = col && plane_form(plan, d);
+    const bool planes = col && plane_form(plan, d) && planes_pay(plan, g);
     if (planes) wv = 1;
     const size_t nimg = (size_t)g.nx * g.ny * g.nz, nprj = (size_t)d.nu * d.nv * nview;
     // column mode: batch items sharing the geometry are backprojected up to 4

@@ -351,3 +351,42 @@ def test_bp_planes_bits_do_not_depend_on_the_run(tuning, case):
     windows = cone.siddon_bp_arbitrary(p, y[:1], *args)
     _say(case, 'voxels that the windows round otherwise: %.2f' % (windows != ref).mean())
     assert (windows != ref).any() and rel_l2(windows, ref) < TOL
+
+
+@pytest.mark.parametrize('case,single,plan', [('thin_1', False, True), ('thin_4', False, True), ('nz_5', True, True),
+                                              ('narrow_4', True, True), ('dense_rows', False, True),
+                                              ('dense_tall', True, True), ('three_rows', False, True)])
+def test_bp_form_by_geometry(oracle, tuning, case, single, plan):
+    """Which column-mode backprojections take the plane form, in single calls
+    (alone and beside another volume) and in a plan: single calls keep the
+    windows for up to 4 slices of wide images and for voxels holding many rows;
+    against the oracle."""
+    import torch
+    from types import SimpleNamespace
+    from ctprojector_amd.batched import ConeBatch, ConeJob
+    from ctprojector_amd.projector.numpy import cone
+    from ctprojector_amd.projector.numpy.ct_projector import ct_projector
+    wide = dict(nx=446, ny=435, dx=0.2, dy=0.2, nu=150, du=1.1)
+    over = {'thin_1': dict(nz=1, **wide), 'thin_4': dict(nz=4, **wide), 'nz_5': dict(nz=5, **wide),
+            'narrow_4': dict(nz=4), 'dense_rows': dict(dv=1.33, nv=90), 'dense_tall': dict(nz=260, dv=1.33, nv=90),
+            'three_rows': dict(dz=1.5, nz=21, dv=0.82, nv=90)}[case]
+    g, args, y = _plane_case(nview=3, B=2, **over)
+    p = g.to(ct_projector())
+    geo = SimpleNamespace(det_center=args[0], det_u=args[1], det_v=args[2], src=args[3])
+
+    def all_ways():
+        b = ConeBatch([ConeJob(p, geo)])
+        b.prj[0].copy_(torch.from_numpy(y[0]))
+        b.backward()
+        return (cone.siddon_bp_arbitrary(p, y[:1], *args), cone.siddon_bp_arbitrary(p, y, *args),
+                b.img[0].cpu().numpy())
+
+    got = all_ways()
+    tuning('cone_bp_planes', 2)
+    windows = all_ways()
+    ref = oracle.siddon_cone_bp(g, y, *args)
+    differs = [bool((a != b).any()) for a, b in zip(got, windows)]
+    _say(case, 'against the oracle %.2e %.2e' % (rel_l2(got[1], ref), rel_l2(got[2], ref[0])), 'not the windows', differs)
+    assert rel_l2(got[1], ref) < TOL and rel_l2(got[2], ref[0]) < TOL
+    assert differs == [single, single, plan]
+    assert np.array_equal(got[0], got[1][:1])
