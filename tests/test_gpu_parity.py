@@ -614,11 +614,11 @@ def test_tomo_window_form(oracle, case):
     print('tomo window', case, e)
     assert max(e) < TOL
     unit, lit = np.zeros_like(img), img.copy()
-    unit[0, 4, 1, 20], lit[0, 4, 1, 20] = 1.0, np.nan
+    at = (0, 4, 14, 12) if case == 'truncated' else (0, 4, 1, 20)   # (within the truncated panel's view)
+    unit[at], lit[at] = 1.0, np.nan
     met = oracle.dd_tomo_fp(g, unit, dc, src) > 1e-4
     bad = np.isnan(tomo.distance_driven_fp(p, lit, dc, src))
-    # (the lit voxel lies beside the truncated panel: no ray meets it)
-    assert met.any() == (case != 'truncated') and bad[met].all() and bad.sum() <= met.sum() + 2
+    assert met.any() and bad[met].all() and bad.sum() <= met.sum() + 2
 
 
 @pytest.mark.parametrize('nz', [1, 2, 3, 4])
@@ -684,3 +684,37 @@ def test_tomo_window_bp_not_finite(oracle, case):
         bad = ~np.isfinite(tomo.distance_driven_bp(_proj(g), np.where(unit > 0, np.float32(value), y), dc, src))
         print('tomo window bp', case, value, int((w > 0).sum()), int(bad.sum()))
         assert (w > 0).sum() > 5 and bad[w > 1e-3 * w.max()].all() and bad.sum() <= (w > 0).sum() + 4
+
+
+@pytest.mark.parametrize('nz', [1, 2, 4, 8])
+@pytest.mark.parametrize('beam', ['fan', 'parallel'])
+def test_dd_row_segments(oracle, tuning, beam, nz):
+    """The one-lane DD projector with 2, 4 and 8 row segments per column (a
+    small launch of 96 rows or more takes 8 by itself), which end inside the
+    window form's stretches of 32 rows: against the oracle, single calls and a
+    batch plan; up to 4 slices in the window form and the walk, 8 in the walk."""
+    import torch
+    from ctprojector_amd.batched import DDBatch, DDJob
+    kw = dict(nx=101, ny=117, nz=nz, dx=1.0, dy=1.0, dz=1.0, cx=1.3, cy=-0.6, nu=97, nv=nz, du=1.37, dv=1.0, off_u=0.31)
+    if beam == 'fan':
+        kw.update(dsd=400.0, dso=240.0, du=2.0)
+    g = Geo(**kw)
+    ang = (np.arange(29) * (2 if beam == 'fan' else 1) * np.pi / 29 + 0.013).astype(np.float32)
+    img = np.random.default_rng(2).uniform(-1, 1, size=[1, nz, g.ny, g.nx]).astype(np.float32)
+    m, ref = (fan, oracle.dd_fan_fp) if beam == 'fan' else (parallel, oracle.dd_par_fp)
+    p, want = _proj(g), ref(g, img, ang)
+    got = {}
+    for segments in (0, 1, 2, 3, 4):        # 0: by rule; 3 and 4: 4 and 8 segments
+        tuning('dd_fp_segments', segments)
+        for mode in (0, 1):
+            tuning('dd_fp_mode', mode)
+            got[segments, mode] = m.distance_driven_fp(p, img, ang)
+        b = DDBatch([DDJob(p, ang, fan=beam == 'fan')])
+        b.img[0].copy_(torch.from_numpy(img[0]).reshape(b.img[0].shape))
+        b.forward()
+        got[segments, 'plan'] = b.prj[0].cpu().numpy().reshape(want.shape)
+        b.close()
+    errs = {k: rel_l2(v, want) for k, v in got.items()}
+    print('dd segments', beam, nz, {k: '%.1e' % e for k, e in errs.items()})
+    assert max(errs.values()) < TOL
+    assert np.array_equal(got[0, 0], got[4, 0])   # eight segments by rule
