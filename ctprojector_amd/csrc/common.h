@@ -73,8 +73,8 @@ __device__ inline float mul_legacy(float a, float b) {
 }
 
 // atan(t) for |t| <= 0.7 ('narrow', uniform across the wavefront), else through
-// the library: t + t z P(z), z = t^2, with P the degree-6 Chebyshev
-// interpolant of (atan(t)/t - 1)/z on [0, 0.5] (within 1 ulp; 9 instructions
+// the library: t + t z P(z), z = t^2, with P the degree-6 truncated
+// Chebyshev series of (atan(t)/t - 1)/z on [0, 0.5] (within 1 ulp; 9 instructions
 // where the general function reduces its argument with a division).
 __device__ inline float fan_atan(float t, bool narrow) {
     if (!narrow) return atanf(t);

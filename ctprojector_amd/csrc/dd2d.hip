@@ -699,7 +699,7 @@ struct FPGroup {               // consecutive views with equal trace flags
 };
 
 // Integral of one lane's line pair over staged pixels [xlo, xlo + width) held
-// in LDS at 'buf' (CHP floats per pixel); the same arithmetic as dd_line.
+// in LDS at 'buf' (CHP floats per pixel); the same arithmetic as footprint().
 template <int CH, int CHP>
 __device__ inline void dd_line_lds(float* acc, const float* buf, int xlo, float x1, float x2, int n, float scale) {
     const float lo = min_f(x1, x2), hi = max_f(x1, x2);
@@ -2028,8 +2028,10 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
             const float ub = tr == 0 ? adj_ucoord<FAN>(xb, yc, V.c, V.s, d, rdu, dso, narrow) : adj_ucoord<FAN>(xc, yb, V.c, V.s, d, rdu, dso, narrow);
             // candidate columns: those whose span [k, k+1] meets [ua, ub],
             // widened by 1e-3 column for the difference between this FP32
-            // projection and the forward projector's FP32 edge lines (about
-            // 1e-5 column); each candidate's weight is then exact
+            // projection and the forward projector's FP32 edge lines (below
+            // 1e-3 up to about 4000 columns; 4e-3 at 16000, where a column met
+            // by less than that at a pixel's edge may be left out); each
+            // candidate's weight is then exact
             const int k0 = max((int)floorf(fminf(ua, ub) - 1e-3f), 0);
             const int k1 = min((int)floorf(fmaxf(ua, ub) + 1e-3f), d.nu - 1);
             const float t = tr == 0 ? (float)iy + 0.5f : (float)ix + 0.5f;
@@ -2058,7 +2060,7 @@ __global__ __launch_bounds__(256) void dd_fp_adjoint_kernel(float* __restrict__ 
                     for (int j = 0; j < CH; j++) q[j] = gp[j];
                 }
                 const float x1 = fmaf(l0.x, t - l1.x, l1.y), x2 = fmaf(l0.y, t - l1.z, l1.w);
-                // the forward projector's IntegralBoxX weight of this pixel (dd_line)
+                // the forward projector's IntegralBoxX weight of this pixel (footprint())
                 const float xl = min_f(x1, x2), xh = max_f(x1, x2);
                 const float a = med_clamp(xl, 0.f, (float)n), b = med_clamp(xh, 0.f, (float)n);
                 const float wt = (fminf(b, lo + 1.f) - fmaxf(a, lo)) * fast_div(l0.z, xh - xl);

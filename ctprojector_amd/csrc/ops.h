@@ -40,12 +40,11 @@ void slices_to_channel_last(float* sino, const float* prj, const SliceRow* rows_
 // prj += A img   (the reference's FP accumulates, cuda/siddon.cu:230)
 void siddon_cone_fp(float* prj, const float* img, const ConeGeomDev& geo, int B, const Grid& g, const Det& d,
                     int nview, hipStream_t stream);
-// img += A^T prj  (exact transpose; synchronises 'stream' at the end)
 // Host copy of a cone geometry on the device (det_center, det_u, det_v, src in
 // a row, 3 nview floats each): gathered on the device, so that the caller
 // waits for one copy instead of four.
 std::vector<float> cone_geometry_to_host(const ConeGeomDev& geo, int nview, hipStream_t stream);
-
+// img += A^T prj  (exact transpose; synchronises 'stream' at the end)
 void siddon_cone_bp(float* img, const float* prj, const ConeGeomDev& geo, const ConeGeomHost& hgeo, int B,
                     const Grid& g, const Det& d, int nview, hipStream_t stream);
 

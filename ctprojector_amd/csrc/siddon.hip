@@ -1379,10 +1379,12 @@ __device__ __forceinline__ void bp_view_col(float* acc, const ConeViewBP& cv, co
 // each plane's crossing ray is split between the two voxels it separates.  One
 // crossing per plane and column instead of two clamped ends per candidate ray
 // and voxel.  Bound by VALU issue like the windows (0.99 instructions per CU
-// cycle): 26 instructions per voxel and view instead of 33, 12.2 -> 9.0 ms at
+// cycle): 26 instructions per voxel and view instead of 33, 12.2 -> 8.9 ms at
 // 256^3 / 720 views, 512 x 384 panel (z-run of 8; 9.6 ms at 4).  Sums kept per
 // plane with the interval lengths folded into the weights take 10% fewer
-// instructions but 106 registers, four wavefronts per SIMD: 9.9 ms.
+// instructions but 106 registers, four wavefronts per SIMD: 9.9 ms.  Parts
+// below a plane computed once for all volumes of a launch: 9.0 ms, and four
+// volumes 2% faster only.
 //
 // Unless MIXED, every plane of the run is above or below the source by at least
 // the view's pm, so that all candidate rays rise or all fall.
@@ -2600,7 +2602,6 @@ void ConePlan::Impl::layout() {
             J.nub = ceil_div(J.d.nu, tu);
             J.ntile = J.nub * ceil_div(J.d.nv, 4 * TV);
         }
-        J.nbx = ceil_div(J.g.nx, 16);
         // plane form: 8 x 8 columns x 4 z-runs per block; windows: 16 x 16 columns x a z-run
         J.nbx = ceil_div(J.g.nx, J.wv == 0 ? 8 : 16);
         J.nby = ceil_div(J.g.ny, J.wv == 0 ? 8 : 16);
