@@ -401,3 +401,39 @@ def test_bp_form_by_geometry(oracle, tuning, case, single, plan):
     assert rel_l2(got[1], ref) < TOL and rel_l2(got[2], ref[0]) < TOL
     assert differs == [single, single, plan]
     assert np.array_equal(got[0], got[1][:1])
+
+
+def test_bp_plan_of_mixed_widths(oracle, tuning):
+    """A batch plan whose jobs have candidate windows of 1 to 4 columns (one
+    launch over all of them, compiled for the widest) and one job in the
+    windows form: every image the same bit for bit as from a plan of that job
+    alone and from one launch per width, and near the oracle's."""
+    import torch
+    from types import SimpleNamespace
+    from ctprojector_amd.batched import ConeBatch, ConeJob
+    from ctprojector_amd.projector.numpy.ct_projector import ct_projector
+    sizes = [dict(du=3.4, nu=22), dict(), dict(du=1.0, nu=75), dict(du=0.75, nu=100, nz=70),
+             dict(nv=260)]   # (rows that far from the source's height cross a plane by more than one within a voxel)
+    jobs, ys, refs = [], [], []
+    for over in sizes:
+        g, args, y = _plane_case(**over)
+        jobs.append(ConeJob(g.to(ct_projector()), SimpleNamespace(det_center=args[0], det_u=args[1], det_v=args[2], src=args[3])))
+        ys.append(torch.from_numpy(y[0]))
+        refs.append(oracle.siddon_cone_bp(g, y, *args)[0])
+
+    def run(picked):
+        b = ConeBatch([jobs[j] for j in picked])
+        for q, j in zip(b.prj, picked):
+            q.copy_(ys[j])
+        b.backward()
+        return [x.cpu().numpy() for x in b.img]
+
+    every = list(range(len(jobs)))
+    alone = [run([j])[0] for j in every]
+    for launch in (1, 2):
+        tuning('cone_plan_bp_launch', launch)
+        for j, x in enumerate(run(every)):
+            assert np.array_equal(x, alone[j]), (launch, j)
+    errs = [rel_l2(x, r) for x, r in zip(alone, refs)]
+    _say('plan of mixed widths', ['%.1e' % e for e in errs])
+    assert max(errs) < TOL
