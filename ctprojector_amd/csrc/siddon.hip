@@ -1379,11 +1379,11 @@ __device__ __forceinline__ void bp_view_col(float* acc, const ConeViewBP& cv, co
 // each plane's crossing ray is split between the two voxels it separates.  One
 // crossing per plane and column instead of two clamped ends per candidate ray
 // and voxel.  Bound by VALU issue like the windows (0.99 instructions per CU
-// cycle): 26 instructions per voxel and view instead of 33, 12.2 -> 8.9 ms at
-// 256^3 / 720 views, 512 x 384 panel (z-run of 8; 9.6 ms at 4).  Sums kept per
+// cycle): 26 instructions per voxel and view instead of 33, 12.2 -> 8.5 ms at
+// 256^3 / 720 views, 512 x 384 panel (z-run of 8; 9.4 ms at 4).  Sums kept per
 // plane with the interval lengths folded into the weights take 10% fewer
 // instructions but 106 registers, four wavefronts per SIMD: 9.9 ms.  Parts
-// below a plane computed once for all volumes of a launch: 9.0 ms, and four
+// below a plane computed once for all volumes of a launch: 1% slower, and four
 // volumes 2% faster only.
 //
 // Unless MIXED, every plane of the run is above or below the source by at least
@@ -1730,21 +1730,31 @@ __device__ __forceinline__ void bp_planes_block(PlaneShare<WU>& sh, float* __res
     }
 }
 
+// Four volumes with windows of two columns: five wavefronts per SIMD at 4 spilled
+// registers (110 and four without the bound: 256^3 / 90 views 3.83 -> 3.75 ms).
 template <int WU, int NZR, int NB>
-__global__ __launch_bounds__(256) void siddon_cone_bp_planes_kernel(float* __restrict__ img, long istride, WTabs wtab,
-                                                                    const float2* __restrict__ utab,
-                                                                    const float* __restrict__ qtab,
-                                                                    const ConeViewBP* __restrict__ views, int nview,
-                                                                    Grid g, int nu, int nv) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 4 && WU == 2 ? 5 : 1)))
+void siddon_cone_bp_planes_kernel(float* __restrict__ img, long istride, WTabs wtab, const float2* __restrict__ utab,
+                                  const float* __restrict__ qtab, const ConeViewBP* __restrict__ views, int nview,
+                                  Grid g, int nu, int nv) {
     __shared__ PlaneShare<WU> sh;
-    bp_planes_block<WU, NZR, NB>(sh, img, istride, wtab, utab, qtab, views, nview, g, nu, nv, blockIdx.x, blockIdx.y,
-                                 blockIdx.z);
+    // Blocks are dealt to the 8 XCDs in turn: XCD i takes the i-th eighth of the
+    // blocks (z slowest), so that its L2 holds a view's rows of that height only
+    // (256^3: one volume / 720 views 8.9 -> 8.5 ms, four / 90 views 4.00 -> 3.83,
+    // where the windows take 3.69).
+    const int per = gridDim.x >> 3, b = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    const int nbx = (g.nx + 7) / 8, nby = (g.ny + 7) / 8;
+    const int bz = b / (nbx * nby), xy = b - bz * nbx * nby, by = xy / nbx;
+    if (bz * 4 * NZR >= g.nz) return;   // (uniform: the last eighth's remainder)
+    bp_planes_block<WU, NZR, NB>(sh, img, istride, wtab, utab, qtab, views, nview, g, nu, nv, xy - by * nbx, by, bz);
 }
 
 template <int WU, int NZR, int NB>
 static void launch_bp_planes_n(float* img, long istride, const WTabs& wtab, const float2* utab, const float* qtab,
                                const ConeViewBP* views, int nview, const Grid& g, const Det& d, hipStream_t stream) {
-    dim3 block(256), grid(ceil_div(g.nx, 8), ceil_div(g.ny, 8), ceil_div(g.nz, 4 * NZR));
+    const long blocks = (long)ceil_div(g.nx, 8) * ceil_div(g.ny, 8) * ceil_div(g.nz, 4 * NZR);
+    if (blocks > 0x7ffffff0L) fail("cone backprojection: too many blocks per launch");
+    dim3 block(256), grid(8 * (unsigned)ceil_div(blocks, 8));
     TimedLaunch t("siddon_cone_bp", stream);
     siddon_cone_bp_planes_kernel<WU, NZR, NB><<<grid, block, 0, stream>>>(img, istride, wtab, utab, qtab, views, nview,
                                                                           g, d.nu, d.nv);
@@ -1756,8 +1766,8 @@ static void launch_bp_planes(float* img, long istride, int nb, const WTabs& wtab
                              const float* qtab, const ConeViewBP* views, int nview, const Grid& g, const Det& d,
                              hipStream_t stream) {
     // Runs of 8 slices for one volume share a run's ends among more voxels
-    // (256^3 / 720 views: 9.3 against 10.1 ms; 128^3 / 180: kernel 318 against
-    // 409 us), where blocks of four such runs are mostly full and number at
+    // (256^3 / 720 views: 9.0 against 9.85 ms; 128^3 / 180: kernel 313 against
+    // 378 us), where blocks of four such runs are mostly full and number at
     // least four a CU (256^2 x 48 / 360 views 1.09 against 1.04 ms, 96^3 / 180
     // 365 against 332 us: runs of 4); runs of 2 where four of them hold the
     // volume (512^2 x 6 / 180: 460 against 483 us).  A voxel's bits are the same
