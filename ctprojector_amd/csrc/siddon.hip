@@ -583,7 +583,8 @@ struct alignas(16) ConeViewBP {
     float pm;               // planes at least this far from the source are crossed by rays of one slope sign
     int extra;              // most rows that can lie wholly within one voxel, less one
     int flip;               // rows are counted from the last one (det_v points down)
-    float pad0, pad1, pad2;
+    int zs;                 // first plane that is not below the source
+    float pad0, pad1;
 };
 
 // Plane form of the column mode: rows staged per view, and most planes of a block.
@@ -745,7 +746,8 @@ static ConeBPPlan make_cone_bp_plan(const ConeGeomHost& h, const Grid& g, const 
         cv.pm = (float)(1.01 * tmax / std::max(ka, 1e-30));
         cv.extra = (int)std::min(1e6, std::ceil(ka / tmin + slack) - 1);
         if (cv.extra > 3) plan.planes = false;
-        cv.pad0 = cv.pad1 = cv.pad2 = 0;
+        cv.zs = (int)std::min(1e9, std::max(-1e9, std::ceil((double)cv.sz)));
+        cv.pad0 = cv.pad1 = 0;
     }
     plan.wu = (int)std::floor(wmax_u) + 1;
     plan.wv = (int)std::floor(wmax_v) + 1;
@@ -1404,14 +1406,14 @@ struct PlaneRun {
     float g, c;            // row coordinate of the plane at height z: c + z g at the end of the span where it is lowest
     float g1, c1;          // (MIXED: for the planes on the other side of the source: c1 + z g1)
     bool above;            // the run's first plane is not below the source
+    int zs;                // the run's first such plane (as an index into the run)
     int wb;                // byte offset of the weight of row -2^22 in the lane's first column
     int stride;            // bytes per row
     unsigned qb;           // LDS address of the staged row table's (biased) row 0
 
-    // first row not wholly below the plane at height z, biased
-    template <bool MIXED>
-    __device__ __forceinline__ float row(float z) const {
-        const bool other = MIXED && (z >= sz) != above;
+    // first row not wholly below the plane at height z, biased; other (uniform):
+    // that plane is not on the side of the run's first
+    __device__ __forceinline__ float row(float z, bool other) const {
         return fmaf(z, other ? g1 : g, other ? c1 : c) + kRowBias;
     }
 };
@@ -1433,7 +1435,7 @@ __device__ __forceinline__ void bp_planes_run(float* acc, const __amdgpu_buffer_
     for (int k = 0; k <= NZR; k++) {
         // rows below 0 and above nv - 1 weigh nothing: their loads are out of
         // the buffers' range and return 0
-        const float rf = R.template row<MIXED>(z[k]);
+        const float rf = R.row(z[k], MIXED && k > 0 && (k >= R.zs) != R.above);
         const int r = __float_as_int(rf);
         fresh[k] = k > 0 && rf != last;
         last = rf;
@@ -1481,10 +1483,10 @@ __device__ __forceinline__ void bp_planes_run(float* acc, const __amdgpu_buffer_
 template <int WU, int NZR, int NB, bool MIXED>
 __device__ __forceinline__ void bp_planes_more(float* acc, const __amdgpu_buffer_rsrc_t* rw, const PlaneColumn<WU>& P,
                                                const PlaneRun& R, const float* z, int extra) {
-    int last = __float_as_int(R.template row<MIXED>(z[0]));
+    int last = __float_as_int(R.row(z[0], false));
 #pragma unroll
     for (int k = 1; k <= NZR; k++) {
-        const int r = __float_as_int(R.template row<MIXED>(z[k]));
+        const int r = __float_as_int(R.row(z[k], MIXED && k > 0 && (k >= R.zs) != R.above));
         const int more = r - last - 1;
         last = r;
         if (__any(more > 0))
@@ -1536,18 +1538,19 @@ __device__ __forceinline__ void bp_planes_column(PlaneColumn<WU>& P, const ConeV
 template <int WU, int NZR, int NB>
 __device__ __forceinline__ void bp_view_planes(float* acc, const ConeViewBP& cv, const PlaneColumn<WU>& P,
                                                const float* const* wt, const float* __restrict__ qrow, int rbase,
-                                               int nu, int nv, const float* z) {
+                                               int nu, int nv, int iz0, const float* z) {
     __amdgpu_buffer_rsrc_t rw[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++)
         rw[b] = __builtin_amdgcn_make_buffer_rsrc((void*)wt[b], (short)0, 4 * nu * nv, 0x00020000);
-    const bool above = z[0] >= cv.sz;                                         // (uniform)
+    const bool above = iz0 >= cv.zs;                                          // (uniform)
     // the candidate rays of planes near the source's height may rise or fall
     const bool mixed = z[0] - cv.sz < cv.pm && z[NZR] - cv.sz > -cv.pm;
     const float g1 = P.v[2 * WU], g0 = P.v[2 * WU + 1];
     PlaneRun R;
     R.sz = cv.sz;
     R.above = above;
+    R.zs = cv.zs - iz0;
     R.g = above ? g1 : g0;
     R.g1 = above ? g0 : g1;
     R.c = fmaf(-cv.sz, R.g, cv.v0);
@@ -1592,7 +1595,7 @@ __device__ float bp_planes_voxel(const float* __restrict__ wtab, const float2* _
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             p[k] = (float)(iz + k) - cv.sz;
-            const float z = (float)(iz + k), g = z >= cv.sz ? g1 : g0;
+            const float z = (float)(iz + k), g = iz + k >= cv.zs ? g1 : g0;
             first[k] = (int)((fmaf(z, g, fmaf(-cv.sz, g, cv.v0)) + kRowBias) - kRowBias);
         }
         for (int r = max(first[0], 0); r <= min(first[1], nv - 1); r++) {
@@ -1703,21 +1706,23 @@ __device__ __forceinline__ void bp_planes_block(PlaneShare<WU>& sh, float* __res
 #pragma unroll
             for (int b = 0; b < NB; b++) wt[b] = wtab.p[b] + view * nuv;
             bp_view_planes<WU, NZR, NB>(acc, cv, P, wt, sh.q[buf][t], __builtin_amdgcn_readfirstlane(sh.rbase[buf][t]),
-                                        nu, nv, z);
+                                        nu, nv, iz0, z);
         }
     }
     if (ix >= g.nx || iy >= g.ny) return;
-    unsigned bad = 0;   // NaN sums, by k * NB + b
+    unsigned bad = 0;   // NaN sums, by k * NB + b: summed again below
+#pragma unroll
+    for (int i = 0; i < NZR * NB; i++) {
+        if (!__builtin_isnan(acc[i])) continue;
+        if (iz0 + i / NB < g.nz) bad |= 1u << i;
+        acc[i] = 0.f;
+    }
 #pragma unroll
     for (int k = 0; k < NZR; k++) {
         const int iz = iz0 + k;
         if (iz < g.nz)
 #pragma unroll
-            for (int b = 0; b < NB; b++) {
-                const float a = acc[k * NB + b];
-                if (__builtin_isnan(a)) bad |= 1u << (k * NB + b);
-                else img[b * istride + ((size_t)iz * g.ny + iy) * g.nx + ix] += a;
-            }
+            for (int b = 0; b < NB; b++) img[b * istride + ((size_t)iz * g.ny + iy) * g.nx + ix] += acc[k * NB + b];
     }
     while (bad != 0) {
         const int i = __builtin_ctz(bad), iz = iz0 + i / NB, b = i % NB;
@@ -2823,11 +2828,15 @@ ConePlan::ConePlan(const std::vector<ConeJobSpec>& specs, bool autotune) : impl_
     if (mode != 0 && mode != 1) fail("cone_fp_mode must be 0 or 1");
     P.tu = mode == 0 ? 0 : tuning_get("cone_fp_tile_u", 32);
     P.order = fp_xcd_order(mode);
-    // plane form's z-run, as launch_bp_planes chooses it, over all jobs (twelve
-    // jobs of 48^3 to 96^3: plan 1.26 ms with runs of 8, 1.28 with 4; four jobs of
-    // 40^3 to 96^3, 682 blocks of runs of 8: 236 us against 190; four jobs of
-    // 128^2 x 2: 207 us with runs of 2, 225 with 4)
+    // plane form's z-run over all jobs: 8 where blocks are mostly full and many,
+    // nine a CU for the kernel of mixed widths (120 registers at a run of 8, four
+    // wavefronts per SIMD, against five; twelve jobs of 48^3 to 96^3, 2796 blocks:
+    // backward 591 us with runs of 8, 612 with 4; ten jobs, 1973 blocks, 535
+    // against 521), four a CU for one width (three jobs of 96^3: 342 against 366),
+    // 2 for up to 8 slices (four jobs of 128^2 x 2: 207 against 225), else 4
     long slices = 0, held = 0, tallest = 0;
+    int widths = 0;
+    for (const Impl::BPGroup& G : P.groups) widths += G.wv == 0;
     for (const ConeJobDev& J : P.jobs)
         if (J.wv == 0) {
             const long tiles = (long)ceil_div(J.g.nx, 8) * ceil_div(J.g.ny, 8);
@@ -2835,9 +2844,8 @@ ConePlan::ConePlan(const std::vector<ConeJobSpec>& specs, bool autotune) : impl_
             held += tiles * 32 * ceil_div(J.g.nz, 32);
             tallest = std::max(tallest, (long)J.g.nz);
         }
-    P.nzr = tuning_get("cone_bp_zrun", 4 * slices > 3 * held && held / 32 >= 4 * 256 ? 8
-                                       : tallest > 0 && tallest <= 8                 ? 2
-                                                                                     : 4);
+    const bool many = 4 * slices > 3 * held && held / 32 >= (widths > 1 ? 9 : 4) * 256;
+    P.nzr = tuning_get("cone_bp_zrun", many ? 8 : tallest > 0 && tallest <= 8 ? 2 : 4);
     if (P.tu != 0 && P.tu != 8 && P.tu != 16 && P.tu != 32 && P.tu != 64)
         fail("cone_fp_tile_u must be 8, 16, 32 or 64");
     if (P.nzr != 2 && P.nzr != 4 && P.nzr != 8) fail("cone plan: cone_bp_zrun must be 2, 4 or 8");
