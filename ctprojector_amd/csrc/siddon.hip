@@ -1381,8 +1381,8 @@ __device__ __forceinline__ void bp_view_col(float* acc, const ConeViewBP& cv, co
 // each plane's crossing ray is split between the two voxels it separates.  One
 // crossing per plane and column instead of two clamped ends per candidate ray
 // and voxel.  Bound by VALU issue like the windows (0.99 instructions per CU
-// cycle): 26 instructions per voxel and view instead of 33, 12.2 -> 8.5 ms at
-// 256^3 / 720 views, 512 x 384 panel (z-run of 8; 9.4 ms at 4).  Sums kept per
+// cycle): 26 instructions per voxel and view instead of 33, 12.2 -> 8.3 ms at
+// 256^3 / 720 views, 512 x 384 panel (z-run of 8; 9.3 ms at 4).  Sums kept per
 // plane with the interval lengths folded into the weights take 10% fewer
 // instructions but 106 registers, four wavefronts per SIMD: 9.9 ms.  Parts
 // below a plane computed once for all volumes of a launch: 1% slower, and four
@@ -1479,28 +1479,47 @@ __device__ __forceinline__ void bp_planes_run(float* acc, const __amdgpu_buffer_
     }
 }
 
-// Rows wholly inside a voxel besides r_{k+1} (where a voxel may hold more than one).
+// Rows wholly inside a voxel besides r_{k+1} (where a voxel may hold more than
+// one), four planes at a time: their loads are issued together, with offsets
+// beyond the buffer, which load 0, for lanes without such a row (runs of 8, 1.3
+// rows per voxel height, 128^2 x 128 / 180 views: 656 us plane by plane, 620 so).
 template <int WU, int NZR, int NB, bool MIXED>
 __device__ __forceinline__ void bp_planes_more(float* acc, const __amdgpu_buffer_rsrc_t* rw, const PlaneColumn<WU>& P,
                                                const PlaneRun& R, const float* z, int extra) {
+    constexpr int G = NB >= 4 ? 1 : NZR < 4 ? NZR : 4;   // (four volumes: one at a time, for the registers)
     int last = __float_as_int(R.row(z[0], false));
 #pragma unroll
-    for (int k = 1; k <= NZR; k++) {
-        const int r = __float_as_int(R.row(z[k], MIXED && k > 0 && (k >= R.zs) != R.above));
-        const int more = r - last - 1;
-        last = r;
-        if (__any(more > 0))
-            for (int e = 1; e <= extra; e++) {
+    for (int k0 = 0; k0 < NZR; k0 += G) {
+        int off[G], more[G];
+        bool some = false;
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            const int k = k0 + i + 1;
+            const int r = __float_as_int(R.row(z[k], MIXED && (k >= R.zs) != R.above));
+            off[i] = __mul24(r, R.stride) + R.wb;
+            more[i] = r - last - 1;
+            last = r;
+            some = some || more[i] > 0;
+        }
+        if (!__any(some)) continue;
+        for (int e = 1; e <= extra; e++) {
+            float x[G][NB][WU];
+#pragma unroll
+            for (int i = 0; i < G; i++) {
+                const int at = e <= more[i] ? off[i] - e * R.stride : (int)0x80000000;
+#pragma unroll
+                for (int b = 0; b < NB; b++) load_floats<WU>(x[i][b], rw[b], at, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < G; i++)
 #pragma unroll
                 for (int b = 0; b < NB; b++) {
-                    float x[WU];
-                    load_floats<WU>(x, rw[b], __mul24(r - e, R.stride) + R.wb, 0);
                     float f = 0.f;
 #pragma unroll
-                    for (int j = 0; j < WU; j++) f = fmaf(x[j], P.v[2 * j + 1] - P.v[2 * j], f);
-                    acc[(k - 1) * NB + b] += e <= more ? f : 0.f;
+                    for (int j = 0; j < WU; j++) f = fmaf(x[i][b][j], P.v[2 * j + 1] - P.v[2 * j], f);
+                    acc[(k0 + i) * NB + b] += f;
                 }
-            }
+        }
     }
 }
 
@@ -1735,22 +1754,28 @@ __device__ __forceinline__ void bp_planes_block(PlaneShare<WU>& sh, float* __res
     }
 }
 
+// Chunks of blocks dealt to the XCDs, for nbz blocks along z: quarters of a layer,
+// or eighths of all blocks where the layers are few.
+__host__ __device__ inline int plane_chunks(int nbz) { return 8 * (nbz >= 4 ? nbz / 2 : 1); }
+
 // Four volumes with windows of two columns: five wavefronts per SIMD at 4 spilled
-// registers (110 and four without the bound: 256^3 / 90 views 3.83 -> 3.75 ms).
+// registers (110 and four without the bound: 256^3 / 720 views 31.9 -> 31.0 ms).
 template <int WU, int NZR, int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 4 && WU == 2 ? 5 : 1)))
 void siddon_cone_bp_planes_kernel(float* __restrict__ img, long istride, WTabs wtab, const float2* __restrict__ utab,
                                   const float* __restrict__ qtab, const ConeViewBP* __restrict__ views, int nview,
                                   Grid g, int nu, int nv) {
     __shared__ PlaneShare<WU> sh;
-    // Blocks are dealt to the 8 XCDs in turn: XCD i takes the i-th eighth of the
-    // blocks (z slowest), so that its L2 holds a view's rows of that height only
-    // (256^3: one volume / 720 views 8.9 -> 8.5 ms, four / 90 views 4.00 -> 3.83,
-    // where the windows take 3.69).
-    const int per = gridDim.x >> 3, b = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    // Blocks are dealt to the 8 XCDs in turn.  XCD i takes chunks i, i + 8, .. of
+    // plane_chunks() chunks of consecutive blocks (z slowest), so that its L2 holds
+    // a view's rows of one height only, and every XCD meets several heights: the
+    // runs near the source's take longer.  (256^3 / 720 views, four volumes: 33.3
+    // ms in plain order, 33.5 with one chunk per XCD, 31.0 so.)
     const int nbx = (g.nx + 7) / 8, nby = (g.ny + 7) / 8;
+    const int per = (int)gridDim.x / plane_chunks((g.nz + 4 * NZR - 1) / (4 * NZR)), at = (int)(blockIdx.x >> 3);
+    const int b = (at / per * 8 + (int)(blockIdx.x & 7)) * per + at % per;
     const int bz = b / (nbx * nby), xy = b - bz * nbx * nby, by = xy / nbx;
-    if (bz * 4 * NZR >= g.nz) return;   // (uniform: the last eighth's remainder)
+    if (bz * 4 * NZR >= g.nz) return;   // (uniform: the last chunk's remainder)
     bp_planes_block<WU, NZR, NB>(sh, img, istride, wtab, utab, qtab, views, nview, g, nu, nv, xy - by * nbx, by, bz);
 }
 
@@ -1758,8 +1783,9 @@ template <int WU, int NZR, int NB>
 static void launch_bp_planes_n(float* img, long istride, const WTabs& wtab, const float2* utab, const float* qtab,
                                const ConeViewBP* views, int nview, const Grid& g, const Det& d, hipStream_t stream) {
     const long blocks = (long)ceil_div(g.nx, 8) * ceil_div(g.ny, 8) * ceil_div(g.nz, 4 * NZR);
-    if (blocks > 0x7ffffff0L) fail("cone backprojection: too many blocks per launch");
-    dim3 block(256), grid(8 * (unsigned)ceil_div(blocks, 8));
+    if (blocks > 0x7f000000L) fail("cone backprojection: too many blocks per launch");
+    const int chunks = plane_chunks(ceil_div(g.nz, 4 * NZR));
+    dim3 block(256), grid((unsigned)chunks * (unsigned)ceil_div(blocks, chunks));
     TimedLaunch t("siddon_cone_bp", stream);
     siddon_cone_bp_planes_kernel<WU, NZR, NB><<<grid, block, 0, stream>>>(img, istride, wtab, utab, qtab, views, nview,
                                                                           g, d.nu, d.nv);
@@ -1771,14 +1797,14 @@ static void launch_bp_planes(float* img, long istride, int nb, const WTabs& wtab
                              const float* qtab, const ConeViewBP* views, int nview, const Grid& g, const Det& d,
                              hipStream_t stream) {
     // Runs of 8 slices for one volume share a run's ends among more voxels
-    // (256^3 / 720 views: 9.0 against 9.85 ms; 128^3 / 180: kernel 313 against
-    // 378 us), where blocks of four such runs are mostly full and number at
-    // least four a CU (256^2 x 48 / 360 views 1.09 against 1.04 ms, 96^3 / 180
-    // 365 against 332 us: runs of 4); runs of 2 where four of them hold the
-    // volume (512^2 x 6 / 180: 460 against 483 us).  A voxel's bits are the same
-    // in all.
+    // (256^3 / 720 views: call 8.5 against 9.8 ms; 128^3 / 180: kernel 302 against
+    // 378 us), where blocks of four such runs are at least seven eighths full and
+    // number four a CU (256^2 x 48 / 360 views 1.09 against 1.04 ms, 160^2 x 100
+    // with 1.3 rows per voxel height 866 against 748 us, 96^3 / 180 365 against 332:
+    // runs of 4); runs of 2 where four of them hold the volume (512^2 x 6 / 180:
+    // 460 against 483 us).  A voxel's bits are the same in all.
     const long span = 32L * ceil_div(g.nz, 32);   // slices of the blocks of runs of 8
-    const bool full = 4L * g.nz > 3 * span && (long)ceil_div(g.nx, 8) * ceil_div(g.ny, 8) * (span / 32) >= 4 * 256;
+    const bool full = 8L * g.nz >= 7 * span && (long)ceil_div(g.nx, 8) * ceil_div(g.ny, 8) * (span / 32) >= 4 * 256;
     const int nzr = tuning_get("cone_bp_zrun", nb > 1 ? 4 : full ? 8 : g.nz <= 8 ? 2 : 4);
     if (nb == 4 && nzr == 4) return launch_bp_planes_n<WU, 4, 4>(img, istride, wtab, utab, qtab, views, nview, g, d, stream);
     if (nb == 2 && nzr == 4) return launch_bp_planes_n<WU, 4, 2>(img, istride, wtab, utab, qtab, views, nview, g, d, stream);
