@@ -1922,14 +1922,15 @@ static bool plane_form(const ConeBPPlan& plan, const Det& d) {
 //   16 x 16 (three blocks a CU): most wavefronts of a plane block have no
 //   slice to work on (448^2 x 4 / 180 views: windows 302 us, planes 368; 512^2
 //   302 against 447; but 384^2 x 4, 576 blocks, 418 against 363);
-// - voxels that often hold whole rows besides the crossing ones, which the
-//   plane form adds one by one.  Windows of two rows: more than 1.25 rows per
-//   voxel height, and rows that differ so much among a block's columns that some
-//   column nearly always has one (1.38 rows, spread 3.0, 200^3 / 90 views:
-//   windows 901 us, planes 974; 1.33 rows, spread 2.1, 160^2 x 128: 526 against
-//   461; 1.28 rows, spread 2.6, 200^3: 896 against 919).  Windows of four rows:
-//   three such rows (200^2 x 128 / 180 views 2.18 against 2.36 ms; with two,
-//   2.26 against 1.87).
+// - voxels that often hold whole rows besides the crossing ones, each a further
+//   load for every volume.  Windows of two rows: more than 1.25 rows per voxel
+//   height, and rows that differ so much among a block's columns that some column
+//   nearly always has one (1.38 rows, spread 3.0, 200^3 / 90 views: windows 0.90
+//   ms, planes 0.92 to 0.97; two volumes 1.39 against 1.74, four 2.29 against 3.12;
+//   1.33 rows, spread 2.1, 160^2 x 128: one volume 0.53 against 0.45).  Windows of
+//   four rows: three such rows (200^2 x 128 / 180 views: one volume 2.18 against
+//   1.98 ms, but two 3.35 against 3.94 and four 5.63 against 7.73; with two such
+//   rows 2.26 against 1.58, 3.45 against 3.13 and 5.73 against 6.11).
 // The rule reads the geometry alone, never how many volumes share a launch:
 // a volume comes out the same alone and beside others.
 static bool planes_pay(const ConeBPPlan& plan, const Grid& g) {
